@@ -249,10 +249,15 @@ int pd_set_timing(pd_sim* s, int level);
  * periodic ghosts (default 4096; more are allocated when a substep needs them);
  * "timing_every" = N records timing events only on substeps 0, N, 2N, ...
  * after pd_set_timing (default 1), which bounds the events' host cost; "velocity_loop_lds" = 1
- * (default) lets a one-workgroup velocity loop of at most 8192 rows keep the velocities of up
- * to "velocity_loop_lds_bodies" of its bodies in LDS (default and maximum 2400; the others stay
- * in global memory) when its rows touch at most "velocity_loop_lds_keys" distinct bodies
- * (default and maximum 12288), 0 keeps them all in global memory; "vsweep_waves" = 3 (default)
+ * (default) runs a velocity loop in one launch over a partition of the bodies, their velocities in
+ * LDS, up to "velocity_loop_lds_bodies" of them per workgroup (default and maximum 2400, which
+ * stands for all that fit; the others stay in global memory), 0 leaves it to the one-workgroup
+ * loop and the launches per colour; a "velocity_loop_lds_keys" below its default and maximum
+ * 12288 makes a loop whose rows may have more distinct bodies leave that launch at its check-in
+ * (one workgroup then runs the loop from global memory); "partition_rows" (default 256; 0 off,
+ * as is block_solver_rows 0): the rows per workgroup of the partitioned velocity and position
+ * loops, four times as many for a loop in one workgroup; "partition_workgroups" (default 224, at
+ * most 256): the most workgroups of one; "vsweep_waves" = 3 (default)
  * or 4 selects the per-colour PGS sweep compiled for that many waves per SIMD (4: at most 128
  * VGPRs, with some register spilling); "velocity_pack_bodies" = 1 (default) lets the per-colour
  * velocity launches read each body's velocity and constants from one 128-byte record packed for

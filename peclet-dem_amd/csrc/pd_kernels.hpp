@@ -2420,32 +2420,23 @@ __device__ __forceinline__ void addVW(Body64& b, d3 dv, d3 dw) {
   b.w.z += dw.z;
 }
 
-// Where a velocity row finds its bodies' velocities: the global array (GBodies), or a copy of
-// the rows' bodies staged in LDS by a one-workgroup sweep loop (LBodies: 6 doubles per body,
-// rows hold the two LDS slots).  The arithmetic is the same either way.
+// Where a velocity row finds its bodies' velocities and constants: the separate global arrays
+// (GBodies) or the packed records (PBodies).  The arithmetic is the same either way.
 struct GBodies {
   Body64* vw;
-  __device__ void row(const Dev& D, int k, int2& r, int2& sl) const {
-    r = D.vAB[k];
-    sl = make_int2(0, 0);
-  }
-  __device__ Body64 load(int real, int) const { return vw[real]; }
-  __device__ void store(int real, int, const Body64& b) const { vw[real] = b; }
+  __device__ Body64 load(int real) const { return vw[real]; }
+  __device__ void store(int real, const Body64& b) const { vw[real] = b; }
   __device__ BodyC cload(const Dev& D, int real) const { return D.bc[real]; }
 };
 struct PBodies {
   VBody* vb;
-  __device__ void row(const Dev& D, int k, int2& r, int2& sl) const {
-    r = D.vAB[k];
-    sl = make_int2(0, 0);
-  }
-  __device__ Body64 load(int real, int) const {
+  __device__ Body64 load(int real) const {
     Body64 b;
     b.v = vb[real].v;
     b.w = vb[real].w;
     return b;
   }
-  __device__ void store(int real, int, const Body64& b) const {
+  __device__ void store(int real, const Body64& b) const {
     vb[real].v = b.v;
     vb[real].w = b.w;
   }
@@ -2475,45 +2466,6 @@ __global__ void k_vb_unpack(const Dev* __restrict__ Dp, const VBody* vb, int n) 
   b.w = vb[i].w;
   D.vw[i] = b;
 }
-// LDS slot codes of a row's bodies: a body without an LDS slot stays in global memory
-constexpr int VL_GLOBAL = 0xFFFE, VL_NONE = 0xFFFF;
-struct LBodies {
-  double2* bv;             // body s: bv[3s] = (v.x, v.y), bv[3s+1] = (v.z, w.x), bv[3s+2] = (w.y, w.z)
-  const unsigned* slots;   // row k - r0: slot of a | slot of b << 16
-  const int* bodyOf;       // slot -> real body
-  PD_G Body64* vw;         // bodies without a slot
-  int r0;
-  __device__ void row(const Dev& D, int k, int2& r, int2& sl) const {
-    const unsigned p = slots[k - r0];
-    sl.x = (int)(p & 0xFFFFu);
-    sl.y = (int)(p >> 16);
-    if (sl.x == VL_GLOBAL || sl.y == VL_GLOBAL) {
-      r = D.vAB[k];
-    } else {
-      r.x = bodyOf[sl.x];
-      r.y = sl.y != VL_NONE ? bodyOf[sl.y] : -1;
-    }
-  }
-  __device__ Body64 load(int real, int s) const {
-    if (s == VL_GLOBAL) return vw[real];
-    const double2 a = bv[3 * s], b = bv[3 * s + 1], c = bv[3 * s + 2];
-    Body64 o;
-    o.v = make_double4(a.x, a.y, b.x, 0.0);
-    o.w = make_double4(b.y, c.x, c.y, 0.0);
-    return o;
-  }
-  __device__ void store(int real, int s, const Body64& o) const {
-    if (s == VL_GLOBAL) {
-      vw[real] = o;
-      return;
-    }
-    bv[3 * s] = make_double2(o.v.x, o.v.y);
-    bv[3 * s + 1] = make_double2(o.v.z, o.w.x);
-    bv[3 * s + 2] = make_double2(o.w.y, o.w.z);
-  }
-  __device__ BodyC cload(const Dev& D, int real) const { return D.bc[real]; }
-};
-
 // A velocity row's constants as k_vrows lays them out: vN = (Nsum, restitution), vRA = (rAavg,
 // mu), vRB = (rBavg, sgn), vTA = TauA, vTB = (TauB, 1 / points); |Nsum| is recomputed (the same
 // expression k_vrows evaluates).  A one-point row (F_ONE) reads neither vTA nor vTB: its sums are
@@ -2537,7 +2489,7 @@ __device__ __forceinline__ void rowTaus(const Dev& D, int k, unsigned char fl, d
 }
 // warmStartApplyKokkos, src/solver_velocity.hpp:498-605 (one row)
 template <class BS>
-__device__ __forceinline__ void warmApplyRowB(const Dev& D, int k, int2 r, int2 sl, const BS& bs) {
+__device__ __forceinline__ void warmApplyRowB(const Dev& D, int k, int2 r, const BS& bs) {
   const double p = D.vLam[k];
   const double4 lt4 = D.vLamT[k];
   d3 lt = xyz(lt4);
@@ -2556,7 +2508,7 @@ __device__ __forceinline__ void warmApplyRowB(const Dev& D, int k, int2 r, int2 
   const d3 Jlin = scale3(Nsum, lambda);
   const BodyC ca = bs.cload(D, realA);
   const double invMassA = ca.iim.w;
-  Body64 ba = bs.load(realA, sl.x);
+  Body64 ba = bs.load(realA);
   const q4 qA = toq(ca.q);
   const d3 invIA = xyz(ca.iim);
   ba.v.x += Jlin.x * invMassA;
@@ -2574,7 +2526,7 @@ __device__ __forceinline__ void warmApplyRowB(const Dev& D, int k, int2 r, int2 
   if (realB >= 0) {
     cb = bs.cload(D, realB);
     invMassB = cb.iim.w;
-    bb = bs.load(realB, sl.y);
+    bb = bs.load(realB);
     bb.v.x += -Jlin.x * invMassB;
     bb.v.y += -Jlin.y * invMassB;
     bb.v.z += -Jlin.z * invMassB;
@@ -2609,14 +2561,12 @@ __device__ __forceinline__ void warmApplyRowB(const Dev& D, int k, int2 r, int2 
       bb.w.z += dw.z;
     }
   }
-  bs.store(realA, sl.x, ba);
-  if (realB >= 0) bs.store(realB, sl.y, bb);
+  bs.store(realA, ba);
+  if (realB >= 0) bs.store(realB, bb);
 }
 __device__ __forceinline__ void warmApplyRow(const Dev& D, int k) {
   const GBodies g{D.vw};
-  int2 r, sl;
-  g.row(D, k, r, sl);
-  warmApplyRowB(D, k, r, sl, g);
+  warmApplyRowB(D, k, D.vAB[k], g);
 }
 
 // A velocity row's constants in the PGS / GS updates (body masses, inertia and orientation do
@@ -2638,7 +2588,7 @@ __device__ __forceinline__ RowPre rowPre(const Params& P, int realB, d3 Nsum, d3
 }
 // PGSManifoldSweep::solveOne, src/solver_velocity.hpp:641-858 (one row)
 template <class BS>
-__device__ __forceinline__ double pgsRowB(const Dev& D, const Params& P, int k, int2 r, int2 sl,
+__device__ __forceinline__ double pgsRowB(const Dev& D, const Params& P, int k, int2 r,
                           double restVelThreshold, const BS& bs) {
   double amax = 0.0;
   const int realA = r.x, realB = r.y;
@@ -2650,7 +2600,7 @@ __device__ __forceinline__ double pgsRowB(const Dev& D, const Params& P, int k, 
   double invMassB = 0.0;
   d3 invIB{0, 0, 0};
   q4 qB{0, 0, 0, 1};
-  Body64 ba = bs.load(realA, sl.x);
+  Body64 ba = bs.load(realA);
   Body64 bb;
   d3 vB{0, 0, 0}, wB{0, 0, 0};
   const unsigned char fl = D.vFlag[k];
@@ -2665,7 +2615,7 @@ __device__ __forceinline__ double pgsRowB(const Dev& D, const Params& P, int k, 
     invMassB = cb.iim.w;
     invIB = xyz(cb.iim);
     qB = toq(cb.q);
-    bb = bs.load(realB, sl.y);
+    bb = bs.load(realB);
     vB = xyz(bb.v);
     wB = xyz(bb.w);
   } else {
@@ -2803,20 +2753,18 @@ __device__ __forceinline__ double pgsRowB(const Dev& D, const Params& P, int k, 
       }
     }
   }
-  if (dirtyA) bs.store(realA, sl.x, ba);
-  if (dirtyB) bs.store(realB, sl.y, bb);
+  if (dirtyA) bs.store(realA, ba);
+  if (dirtyB) bs.store(realB, bb);
   return amax;
 }
 __device__ __forceinline__ double pgsRow(const Dev& D, const Params& P, int k, double restVelThreshold) {
   const GBodies g{D.vw};
-  int2 r, sl;
-  g.row(D, k, r, sl);
-  return pgsRowB(D, P, k, r, sl, restVelThreshold, g);
+  return pgsRowB(D, P, k, D.vAB[k], restVelThreshold, g);
 }
 
 // solveVelocityColoredGSKokkos one-shot restitution (g = 0), src/solver_velocity.hpp:989-1133
 template <class BS>
-__device__ __forceinline__ double gsRowB(const Dev& D, const Params& P, int k, int2 r, int2 sl,
+__device__ __forceinline__ double gsRowB(const Dev& D, const Params& P, int k, int2 r,
                          double restVelThreshold, const BS& bs) {
   const int realA = r.x, realB = r.y;
   const BodyC ca = bs.cload(D, realA);
@@ -2827,7 +2775,7 @@ __device__ __forceinline__ double gsRowB(const Dev& D, const Params& P, int k, i
   double invMassB = 0.0;
   d3 invIB{0, 0, 0};
   q4 qB{0, 0, 0, 1};
-  Body64 ba = bs.load(realA, sl.x);
+  Body64 ba = bs.load(realA);
   Body64 bb;
   d3 vB{0, 0, 0}, wB{0, 0, 0};
   const unsigned char fl = D.vFlag[k];
@@ -2842,7 +2790,7 @@ __device__ __forceinline__ double gsRowB(const Dev& D, const Params& P, int k, i
     invMassB = cb.iim.w;
     invIB = xyz(cb.iim);
     qB = toq(cb.q);
-    bb = bs.load(realB, sl.y);
+    bb = bs.load(realB);
     vB = xyz(bb.v);
     wB = xyz(bb.w);
   } else {
@@ -2879,7 +2827,7 @@ __device__ __forceinline__ double gsRowB(const Dev& D, const Params& P, int k, i
     ba.w.y += dw.y;
     ba.w.z += dw.z;
   }
-  bs.store(realA, sl.x, ba);
+  bs.store(realA, ba);
   if (realB >= 0) {
     bb.v.x += -Jlin.x * invMassB;
     bb.v.y += -Jlin.y * invMassB;
@@ -2888,15 +2836,13 @@ __device__ __forceinline__ double gsRowB(const Dev& D, const Params& P, int k, i
     bb.w.x += dw.x;
     bb.w.y += dw.y;
     bb.w.z += dw.z;
-    bs.store(realB, sl.y, bb);
+    bs.store(realB, bb);
   }
   return amax;
 }
 __device__ __forceinline__ double gsRow(const Dev& D, const Params& P, int k, double restVelThreshold) {
   const GBodies g{D.vw};
-  int2 r, sl;
-  g.row(D, k, r, sl);
-  return gsRowB(D, P, k, r, sl, restVelThreshold, g);
+  return gsRowB(D, P, k, D.vAB[k], restVelThreshold, g);
 }
 // the same rows on packed body records: RowOf<false> reads vw / bc, RowOf<true> one VBody each
 template <bool PK>
@@ -2913,47 +2859,46 @@ template <>
 struct RowOf<true> {
   __device__ __forceinline__ static void warm(const Dev& D, int k, VBody* vb) {
     const PBodies p{vb};
-    int2 r, sl;
-    p.row(D, k, r, sl);
-    warmApplyRowB(D, k, r, sl, p);
+    warmApplyRowB(D, k, D.vAB[k], p);
   }
   __device__ static double pgs(const Dev& D, const Params& P, int k, double thr, VBody* vb) {
     const PBodies p{vb};
-    int2 r, sl;
-    p.row(D, k, r, sl);
-    return pgsRowB(D, P, k, r, sl, thr, p);
+    return pgsRowB(D, P, k, D.vAB[k], thr, p);
   }
   __device__ static double gs(const Dev& D, const Params& P, int k, double thr, VBody* vb) {
     const PBodies p{vb};
-    int2 r, sl;
-    p.row(D, k, r, sl);
-    return gsRowB(D, P, k, r, sl, thr, p);
+    return gsRowB(D, P, k, D.vAB[k], thr, p);
   }
 };
 
-// computeSideFlagsKokkos, src/solver_velocity.hpp:456-495 (rows are active, non-duplicate)
+// computeSideFlagsKokkos, src/solver_velocity.hpp:456-495 (rows are active, non-duplicate), from
+// the row's flags and its bodies' velocities; the result has the side bits set anew
+__device__ __forceinline__ unsigned char sideFlags(const Dev& D, int2 r, unsigned char fl0,
+                                                   double vn0, d3 vA, d3 vB, d3 gHat,
+                                                   double riseThr, double approachThr) {
+  unsigned char fl = fl0 & (unsigned char)~(F_SIDE1 | F_SIDE2);
+  if (r.y >= 0 && (fl & F_PERSIST) && !(fabs(vn0) > approachThr)) {
+    if ((fl & F_UP) && -dot3(vB, gHat) <= riseThr && D.ground[r.y] > 0)
+      fl |= F_SIDE1;
+    else if ((fl & F_DOWN) && -dot3(vA, gHat) <= riseThr && D.ground[r.x] > 0)
+      fl |= F_SIDE2;
+  }
+  return fl;
+}
 template <class BS>
 __device__ __forceinline__ void sideFlagsRow(const Dev& D, int k, d3 gHat, double riseThr,
                                              double approachThr, const BS& bs) {
-  unsigned char fl = D.vFlag[k] & (unsigned char)~(F_SIDE1 | F_SIDE2);
-  int2 r, sl;
-  bs.row(D, k, r, sl);
-  if (r.y >= 0 && (fl & F_PERSIST) && !(fabs(D.vVn0[k]) > approachThr)) {
-    if ((fl & F_UP) && -dot3(xyz(bs.load(r.y, sl.y).v), gHat) <= riseThr && D.ground[r.y] > 0)
-      fl |= F_SIDE1;
-    else if ((fl & F_DOWN) && -dot3(xyz(bs.load(r.x, sl.x).v), gHat) <= riseThr &&
-             D.ground[r.x] > 0)
-      fl |= F_SIDE2;
-  }
-  D.vFlag[k] = fl;
+  const int2 r = D.vAB[k];
+  const d3 vA = xyz(bs.load(r.x).v);
+  const d3 vB = r.y >= 0 ? xyz(bs.load(r.y).v) : d3{0.0, 0.0, 0.0};
+  D.vFlag[k] = sideFlags(D, r, D.vFlag[k], D.vVn0[k], vA, vB, gHat, riseThr, approachThr);
 }
-// `need` (optional) gates the launch like `run`
 // vb (optional): the stage's packed body records
 __global__ void k_side_flags(const Dev* __restrict__ Dp, int numRows, d3 gHat, double riseThr, double approachThr,
-                             const int* run, const int* need, VBody* vb = nullptr) {
+                             const int* run, VBody* vb = nullptr) {
   const Dev& D = *Dp;
   const int k = gtid();
-  if (k >= numRows || !*run || (need && !*need)) return;
+  if (k >= numRows || !*run) return;
   if (vb)
     sideFlagsRow(D, k, gHat, riseThr, approachThr, PBodies{vb});
   else
@@ -2963,7 +2908,8 @@ __global__ void k_side_flags(const Dev* __restrict__ Dp, int numRows, d3 gHat, d
 // mode: 0 = warm start, 1 = PGS sweep, 2 = one-shot GS sweep
 // ---- device-side loop control: ctl[0..] ints (see pd_sim.hip), sweeps after a stop are no-ops
 enum { CTL_STOP_V = 0, CTL_SWEEPS_V, CTL_STAB_RUN, CTL_STOP_S, CTL_SWEEPS_S, CTL_STOP_P,
-       CTL_SWEEPS_P, CTL_NONE, CTL_VFALLBACK, CTL_COUNT };
+       CTL_SWEEPS_P, CTL_NONE, CTL_PARTS_BUSY, CTL_PARTS_OVER,
+       CTL_PARTS_FAIL, CTL_COUNT };
 __global__ void k_sweep_begin(unsigned long long* bits, const int* stop) {
   if (!*stop) *bits = 0ull;
 }
@@ -2979,9 +2925,7 @@ __global__ void k_sweep_check(unsigned long long* bits, int* stop, int* count, d
   else if (next) *bits = 0ull;
 }
 // stabilization gate (src/sim.hpp:279-283): run iff mode != 0 and the residual exceeds vRestS
-__global__ void k_stab_gate(const unsigned long long* bits, int* ctl, int mode, double vRestS,
-                            const int* need) {
-  if (need && !*need) return;
+__global__ void k_stab_gate(const unsigned long long* bits, int* ctl, int mode, double vRestS) {
   const int run = (mode != 0 && bitsd(*bits) > vRestS) ? 1 : 0;
   ctl[CTL_STAB_RUN] = run;
   ctl[CTL_STOP_S] = run ? 0 : 1;
@@ -3423,35 +3367,23 @@ __global__ __launch_bounds__(VBLOCK_THREADS) void k_vsweep_tail(
   if (mode != 0 && threadIdx.x == 0 && M) atomicMax(D.maxApproachBits, M);
 }
 
-// The sweep loop proper (MODE 1 = PGS, 2 = one-shot GS) over rows whose bodies live in `bs`;
+// The sweep loop proper (MODE 1 = PGS, 2 = one-shot GS) by one workgroup, bodies in global memory;
 // returns after the sweep that meets the stop rule or after `iters` sweeps.
-template <int MODE, class BS>
+template <int MODE>
 __device__ __forceinline__ void vSweepLoop(const Dev& D, const Params& P, const ClassStarts& cs,
-                                           int numColors, int numManifolds, int iters, double thr,
-                                           double stopThr, int* stop, int* count, const BS& bs,
-                                           unsigned long long* sh) {
+                                           int numColors, int iters, double thr, double stopThr,
+                                           int* stop, int* count, unsigned long long* sh) {
   for (int it = 0; it < iters; ++it) {
     unsigned long long m = 0;
     for (int c = 0; c < numColors; ++c) {
       const int b = cs.s[c], e = cs.s[c + 1];
       if (e <= b) continue;
-      if (c == 62) {
-        if (threadIdx.x == 0)
-          for (int k = b; k < e; ++k) {
-            int2 r, sl;
-            bs.row(D, k, r, sl);
-            const unsigned long long a = dbits(MODE == 1 ? pgsRowB(D, P, k, r, sl, thr, bs)
-                                                         : gsRowB(D, P, k, r, sl, thr, bs));
-            m = a > m ? a : m;
-          }
-      } else {
-        for (int k = b + (int)threadIdx.x; k < e; k += blockDim.x) {
-          int2 r, sl;
-          bs.row(D, k, r, sl);
-          const unsigned long long a = dbits(MODE == 1 ? pgsRowB(D, P, k, r, sl, thr, bs)
-                                                       : gsRowB(D, P, k, r, sl, thr, bs));
-          m = a > m ? a : m;
-        }
+      // (the last class may hold rows sharing a body: one thread, in row order)
+      const int step = c == 62 ? 1 : (int)blockDim.x;
+      const int first = c == 62 ? (threadIdx.x == 0 ? b : e) : b + (int)threadIdx.x;
+      for (int k = first; k < e; k += step) {
+        const unsigned long long a = dbits(MODE == 1 ? pgsRow(D, P, k, thr) : gsRow(D, P, k, thr));
+        m = a > m ? a : m;
       }
       __syncthreads();
     }
@@ -3466,194 +3398,29 @@ __device__ __forceinline__ void vSweepLoop(const Dev& D, const Params& P, const 
     }
   }
 }
-// MODE 0 = warm start (one pass), 1 = PGS, 2 = one-shot GS.  `run` and `need` (optional) gate
-// the whole loop; `stop` / `count` / `bits` are the loop's stop flag, sweep counter and residual.
+__device__ __forceinline__ void vWarmPass(const Dev& D, const ClassStarts& cs,
+                                          int numColors) {
+  for (int c = 0; c < numColors; ++c) {
+    const int b = cs.s[c], e = cs.s[c + 1];
+    if (e <= b) continue;
+    const int step = c == 62 ? 1 : (int)blockDim.x;
+    const int first = c == 62 ? (threadIdx.x == 0 ? b : e) : b + (int)threadIdx.x;
+    for (int k = first; k < e; k += step) warmApplyRow(D, k);
+    __syncthreads();
+  }
+}
+// MODE 0 = warm start (one pass), 1 = PGS, 2 = one-shot GS.  `run` (optional) gates the whole loop; `stop` / `count` / `bits` are the loop's stop flag, sweep counter and residual.
 template <int MODE>
 __global__ __launch_bounds__(VBLOCK_THREADS) void k_vsolve_block(
-    const Dev* __restrict__ Dp, Params P, ClassStarts cs, int numColors, int numManifolds, int iters, double thr,
-    double stopThr, int* stop, int* count, const int* run, const int* need) {
+    const Dev* __restrict__ Dp, Params P, ClassStarts cs, int numColors, int iters, double thr,
+    double stopThr, int* stop, int* count, const int* run) {
   const Dev& D = *Dp;
   __shared__ unsigned long long sh[VBLOCK_THREADS / 64];
-  if ((run && !*run) || (need && !*need) || *stop) return;
-  if (MODE == 0) {
-    for (int c = 0; c < numColors; ++c) {
-      const int b = cs.s[c], e = cs.s[c + 1];
-      if (e <= b) continue;
-      if (c == 62) {
-        if (threadIdx.x == 0)
-          for (int k = b; k < e; ++k) warmApplyRow(D, k);
-      } else {
-        for (int k = b + (int)threadIdx.x; k < e; k += blockDim.x) warmApplyRow(D, k);
-      }
-      __syncthreads();
-    }
-    return;
-  }
-  vSweepLoop<MODE>(D, P, cs, numColors, numManifolds, iters, thr, stopThr, stop, count,
-                   GBodies{D.vw}, sh);
-}
-// The velocity loops with their bodies staged in LDS: a colour pass reads and writes the velocities
-// of up to bodyCap (<= VL_BODIES) of the rows' bodies in LDS, the rest in global memory (the
-// row constants stay in global memory, read-only in the loop), and the staged velocities go back
-// to global memory once.  Staging hashes the rows' distinct bodies into LDS (the hash shares the
-// velocity area, which is filled after it); more than VL_ROWS rows or keyCap distinct bodies
-// change nothing and set *fallback = 1 (then k_vsolve_block, gated on it, runs the loop);
-// otherwise *fallback = 0.
-constexpr int VL_ROWS = 8192;
-constexpr int VL_BODIES = 2400;
-constexpr int VL_HASH = 16384;
-static_assert(VL_HASH * (sizeof(int) + sizeof(unsigned short)) <= 3 * VL_BODIES * sizeof(double2),
-              "the staging hash fits in the velocity area");
-static_assert(VL_BODIES < VL_GLOBAL, "LDS body slots");
-constexpr int VL_KEYS = VL_HASH * 3 / 4;  // distinct bodies the hash takes at most
-// open-addressing slot of `body` in an LDS hash of VL_HASH keys (-1: full or, on lookup, absent)
-__device__ __forceinline__ int vlSlot(int* hKey, int* used, int body, bool insert, int keyCap) {
-  unsigned h = ((unsigned)body * 2654435761u) & (VL_HASH - 1);
-  for (int probe = 0; probe < VL_HASH; ++probe) {
-    const int k = hKey[h];
-    if (k == body) return (int)h;
-    if (k == -1) {
-      if (!insert) return -1;
-      if (atomicAdd(used, 1) >= keyCap) return -1;
-      const int old = atomicCAS(&hKey[h], -1, body);
-      if (old == -1 || old == body) return (int)h;
-      atomicSub(used, 1);
-      continue;  // lost the slot to another body: look at it again
-    }
-    h = (h + 1) & (VL_HASH - 1);
-  }
-  return -1;
-}
-// The velocity stage one launch runs on the staged bodies: optionally the warm-start pass, the
-// sweep loop, and optionally the stabilization gate (src/sim.hpp:279-283) followed, for
-// stabilization mode 1, by the side flags and the stabilization loop.
-struct VStage {
-  int warm;  // 1: warm-start pass first
-  int iters;
-  double thr, stopThr;
-  int *stop, *count;
-  int gate;      // 1: stabilization gate after the loop (writes stabRun and stabStop)
-  int stabMode;  // the gate's mode; mode 1 also runs the side flags and the loop
-  int stabIters;
-  double stabThr;
-  int *stabRun, *stabStop, *stabCount;
-  d3 gHat;
-  double riseThr, approachThr;
-};
-template <int MODE>
-__global__ __launch_bounds__(VBLOCK_THREADS) void k_vsolve_lds(
-    const Dev* __restrict__ Dp, Params P, ClassStarts cs, int numColors, int numManifolds,
-    VStage S, int* fallback, int bodyCap, int keyCap) {
-  const Dev& D = *Dp;
-
-  __shared__ unsigned long long sh[VBLOCK_THREADS / 64];
-  __shared__ double2 bv[3 * VL_BODIES];
-  __shared__ int bodyOf[VL_BODIES];
-  __shared__ unsigned slots[VL_ROWS];
-  __shared__ int sUsed, sFail, sDense;
-  int* hKey = reinterpret_cast<int*>(bv);
-  unsigned short* hIdx = reinterpret_cast<unsigned short*>(hKey + VL_HASH);
-  if (*S.stop) return;  // (zero at the start of a substep)
-  const int T = blockDim.x, tid = threadIdx.x;
-  const int r0 = cs.s[0], nRows = cs.s[numColors] - r0;
-  if (nRows > VL_ROWS) {
-    if (tid == 0) *fallback = 1;
-    return;
-  }
-  for (int h = tid; h < VL_HASH; h += T) hKey[h] = -1;
-  if (tid == 0) {
-    sUsed = 0;
-    sFail = 0;
-    sDense = 0;
-  }
-  __syncthreads();
-  for (int q = tid; q < nRows; q += T) {
-    const int2 r = D.vAB[r0 + q];
-    if (vlSlot(hKey, &sUsed, r.x, true, keyCap) < 0) sFail = 1;
-    if (r.y >= 0 && vlSlot(hKey, &sUsed, r.y, true, keyCap) < 0) sFail = 1;
-  }
-  __syncthreads();
-  const bool staged = !sFail;
-  if (tid == 0) *fallback = staged ? 0 : 1;
-  if (!staged) return;
-  // dense LDS slots for the first bodyCap bodies met in hash order, the rest stay global
-  for (int h = tid; h < VL_HASH; h += T) {
-    const int body = hKey[h];
-    if (body < 0) continue;
-    const int s = atomicAdd(&sDense, 1);
-    if (s < bodyCap) {
-      hIdx[h] = (unsigned short)s;
-      bodyOf[s] = body;
-    } else {
-      hIdx[h] = (unsigned short)VL_GLOBAL;
-    }
-  }
-  __syncthreads();
-  for (int q = tid; q < nRows; q += T) {
-    const int2 r = D.vAB[r0 + q];
-    const unsigned sa = hIdx[vlSlot(hKey, &sUsed, r.x, false, keyCap)];
-    const unsigned sb = r.y >= 0 ? hIdx[vlSlot(hKey, &sUsed, r.y, false, keyCap)] : VL_NONE;
-    slots[q] = sa | (sb << 16);
-  }
-  __syncthreads();  // the hash is dead: its area now takes the velocities
-  const int nb = sDense < bodyCap ? sDense : bodyCap;
-  for (int s = tid; s < nb; s += T) {
-    const Body64 g = D.vw[bodyOf[s]];
-    bv[3 * s] = make_double2(g.v.x, g.v.y);
-    bv[3 * s + 1] = make_double2(g.v.z, g.w.x);
-    bv[3 * s + 2] = make_double2(g.w.y, g.w.z);
-  }
-  __syncthreads();
-  const LBodies bs{bv, slots, bodyOf, D.vw, r0};
-  if (S.warm) {
-    for (int c = 0; c < numColors; ++c) {
-      const int b = cs.s[c], e = cs.s[c + 1];
-      if (e <= b) continue;
-      if (c == 62) {
-        if (tid == 0)
-          for (int k = b; k < e; ++k) {
-            int2 r, sl;
-            bs.row(D, k, r, sl);
-            warmApplyRowB(D, k, r, sl, bs);
-          }
-      } else {
-        for (int k = b + tid; k < e; k += T) {
-          int2 r, sl;
-          bs.row(D, k, r, sl);
-          warmApplyRowB(D, k, r, sl, bs);
-        }
-      }
-      __syncthreads();
-    }
-  }
-  vSweepLoop<MODE>(D, P, cs, numColors, numManifolds, S.iters, S.thr, S.stopThr, S.stop, S.count,
-                   bs, sh);
-  if (S.gate) {
-    __syncthreads();  // the loop's last residual is in *D.maxApproachBits
-    const int runS = (S.stabMode != 0 && bitsd(*D.maxApproachBits) > S.stabThr) ? 1 : 0;
-    if (tid == 0) {
-      *S.stabRun = runS;
-      *S.stabStop = runS ? 0 : 1;
-    }
-    if (runS && S.stabMode == 1) {
-      for (int k = r0 + tid; k < r0 + nRows; k += T)
-        sideFlagsRow(D, k, S.gHat, S.riseThr, S.approachThr, bs);
-      __syncthreads();
-      vSweepLoop<1>(D, P, cs, numColors, numManifolds, S.stabIters, S.stabThr, S.stabThr,
-                    S.stabStop, S.stabCount, bs, sh);
-    }
-  }
-  __syncthreads();
-  for (int s = tid; s < nb; s += T) {
-    PD_G Body64* g = D.vw + bodyOf[s];
-    const double2 a = bv[3 * s], b = bv[3 * s + 1], c = bv[3 * s + 2];
-    g->v.x = a.x;
-    g->v.y = a.y;
-    g->v.z = b.x;
-    g->w.x = b.y;
-    g->w.y = c.x;
-    g->w.z = c.y;
-  }
+  if ((run && !*run) || *stop) return;
+  if (MODE == 0)
+    vWarmPass(D, cs, numColors);
+  else
+    vSweepLoop<MODE>(D, P, cs, numColors, iters, thr, stopThr, stop, count, sh);
 }
 // ---- stabilization mode 4 ("ordered"), src/sim.hpp:356-397 ---------------------------------
 constexpr int LEVEL_INF = 1 << 28;
@@ -3970,29 +3737,20 @@ __global__ void k_psweep_serial(const Dev* __restrict__ Dp, int rowBegin, int ro
   for (int k = rowBegin; k < rowEnd; ++k) atomicMaxD(D.maxOverlapBits, posRow(D, k));
 }
 
-// position sweeps (XPBD), strict stop: residual < tol
-__global__ __launch_bounds__(BLOCK_SOLVER_THREADS) void k_psolve_block(
-    const Dev* __restrict__ Dp, ClassStarts cs, int numColors, int numContacts, int iters, double tol, int* stop,
-    int* count) {
-  const Dev& D = *Dp;
-  __shared__ unsigned long long sh[BLOCK_SOLVER_THREADS / 64];
-  if (*stop) return;
+// position sweeps (XPBD) by one workgroup, strict stop: residual < tol
+__device__ __forceinline__ void pSweepLoop(const Dev& D, const ClassStarts& cs, int numColors,
+                                           int iters, double tol, int* stop, int* count,
+                                           unsigned long long* sh) {
   for (int it = 0; it < iters; ++it) {
     unsigned long long m = 0;
     for (int c = 0; c < numColors; ++c) {
       const int b = cs.s[c], e = cs.s[c + 1];
       if (e <= b) continue;
-      if (c == 62) {
-        if (threadIdx.x == 0)
-          for (int k = b; k < e; ++k) {
-            const unsigned long long a = dbits(posRow(D, k));
-            m = a > m ? a : m;
-          }
-      } else {
-        for (int k = b + (int)threadIdx.x; k < e; k += blockDim.x) {
-          const unsigned long long a = dbits(posRow(D, k));
-          m = a > m ? a : m;
-        }
+      const int step = c == 62 ? 1 : (int)blockDim.x;
+      const int first = c == 62 ? (threadIdx.x == 0 ? b : e) : b + (int)threadIdx.x;
+      for (int k = first; k < e; k += step) {
+        const unsigned long long a = dbits(posRow(D, k));
+        m = a > m ? a : m;
       }
       __syncthreads();
     }
@@ -4006,6 +3764,14 @@ __global__ __launch_bounds__(BLOCK_SOLVER_THREADS) void k_psolve_block(
       return;
     }
   }
+}
+__global__ __launch_bounds__(BLOCK_SOLVER_THREADS) void k_psolve_block(
+    const Dev* __restrict__ Dp, ClassStarts cs, int numColors, int iters, double tol, int* stop,
+    int* count) {
+  const Dev& D = *Dp;
+  __shared__ unsigned long long sh[BLOCK_SOLVER_THREADS / 64];
+  if (*stop) return;
+  pSweepLoop(D, cs, numColors, iters, tol, stop, count, sh);
 }
 
 // The small colours of one position sweep in one workgroup, then the sweep's stop check: the

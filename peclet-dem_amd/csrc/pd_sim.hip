@@ -26,6 +26,7 @@
 #include "pd_adjoint.hpp"
 #include "pd_hertz.hpp"
 #include "pd_kernels.hpp"
+#include "pd_parts.hpp"
 #include "peclet_dem.h"
 
 using namespace pd;
@@ -189,8 +190,19 @@ struct pd_sim {
   int blockRows = BLOCK_SOLVER_ROWS;
   bool ldsLoop = true;  // one-workgroup velocity loops stage their bodies in LDS when they fit
   bool vsweepWaves4 = false;  // per-colour PGS sweeps compiled for 4 waves per SIMD
-  int ldsBodies = VL_BODIES;  // ... up to this many bodies (the rest stay in global memory)
-  int ldsKeys = VL_KEYS;      // more distinct bodies than this: the global-memory loop
+  // ... up to this many per workgroup (the rest stay in global memory; LDS_BODIES_MAX: all that fit)
+  static constexpr int LDS_BODIES_MAX = 2400;
+  int ldsBodies = LDS_BODIES_MAX;
+  // rows that may have more distinct bodies than this: the loop leaves at its check-in and one
+  // workgroup runs it from global memory (LDS_KEYS_MAX: never)
+  static constexpr int LDS_KEYS_MAX = 12288;
+  int ldsKeys = LDS_KEYS_MAX;
+  // sweep loops over a partition of the bodies (pd_parts.hpp): rows per workgroup (0: off) and the
+  // most workgroups
+  long partRows = 256;
+  int partMax = 224;
+  long partsBusy = 0;       // substeps to go before the partitioned loops are tried again ...
+  long partsBusyNext = 64;  // ... after one found the device busy
   // extra slots reserved by setPositions for periodic ghosts (more are added when needed)
   long slotHeadroom = 4096;
   // the largest scale, cached while no scale is written (every writer clears scaleKnown)
@@ -372,6 +384,14 @@ struct pd_sim {
     HIPCHECK(hipHostGetDevicePointer(&jobP.pinnedDev, jobP.pinned, 0));
     jobV.stream = st;
     jobP.stream = sideStream;
+    for (const void* f : {reinterpret_cast<const void*>(&k_vsolve_lds<1, false>),
+                          reinterpret_cast<const void*>(&k_vsolve_lds<1, true>),
+                          reinterpret_cast<const void*>(&k_vsolve_lds<2, false>),
+                          reinterpret_cast<const void*>(&k_vsolve_lds<2, true>),
+                          reinterpret_cast<const void*>(&k_psolve_lds<false>),
+                          reinterpret_cast<const void*>(&k_psolve_lds<true>)})
+      HIPCHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   std::max(PT_VBODIES * 48, PT_PBODIES * 24)));
     ensureSlots(cap > 0 ? cap : 1, 0);
     // src/sim.hpp:318-321: the multilevel gate mask comes from the environment, default slip
     if (const char* e = std::getenv("PECLET_DEM_ML_GATES")) mlGates = std::atoi(e);
@@ -444,7 +464,7 @@ struct pd_sim {
     hXi.release(); hF.release(); hTA.release(); hTB.release(); hPrevXi.release();
     hRefPos.release(); hXiWall.release(); hWF.release(); hWT.release(); hPrevKeys.release();
     hTab.release();
-    jobV.release(); jobP.release(); redPart.release();
+    jobV.release(); jobP.release(); partsV.release(); partsP.release(); redPart.release();
     ctl.release(); supList.release(); supCnt.release(); hLevel.release(); lvlKey.release(); lvlCnt.release();
     lvlStart.release(); lvlPerm.release(); lvlChanged.release(); lvlBuckets.release();
   }
@@ -1840,20 +1860,149 @@ struct pd_sim {
   }
 
   // One-workgroup velocity sweep loop in global memory (mode 1 PGS, 2 one-shot GS, or 0 the
-  // warm-start pass) over the colour classes vs; `need` (optional) gates it on a device flag.
+  // warm-start pass) over the colour classes vs.
   void vLoop(int mode, const Params& P, const std::vector<int>& vs, int numColors, int iters,
-             double thr, double stopThr, int* stop, int* count, const int* run,
-             const int* need = nullptr) {
+             double thr, double stopThr, int* stop, int* count, const int* run) {
     const ClassStarts cs = classStarts(vs);
     if (mode == 0)
-      k_vsolve_block<0><<<1, VBLOCK_THREADS, 0, st>>>(dD, P, cs, numColors, nm, iters, thr,
-                                                       stopThr, stop, count, run, need);
+      k_vsolve_block<0><<<1, VBLOCK_THREADS, 0, st>>>(dD, P, cs, numColors, iters, thr, stopThr,
+                                                       stop, count, run);
     else if (mode == 1)
-      k_vsolve_block<1><<<1, VBLOCK_THREADS, 0, st>>>(dD, P, cs, numColors, nm, iters, thr,
-                                                       stopThr, stop, count, run, need);
+      k_vsolve_block<1><<<1, VBLOCK_THREADS, 0, st>>>(dD, P, cs, numColors, iters, thr, stopThr,
+                                                       stop, count, run);
     else
-      k_vsolve_block<2><<<1, VBLOCK_THREADS, 0, st>>>(dD, P, cs, numColors, nm, iters, thr,
-                                                       stopThr, stop, count, run, need);
+      k_vsolve_block<2><<<1, VBLOCK_THREADS, 0, st>>>(dD, P, cs, numColors, iters, thr, stopThr,
+                                                       stop, count, run);
+  }
+  // One partition of the rows of a sweep loop (pd_parts.hpp): the velocity rows over the reals, or
+  // the position rows over the slots.
+  struct PartJob {
+    DBuf<PartGrid> grid;
+    DBuf<unsigned long long> mask;
+    DBuf<int> hist, cellStart, partOf, partCnt, partIds, bktCnt, listStart, list;
+    DBuf<int4> bkt, ent;
+    DBuf<int2> rank, nxt;
+    DBuf<double> lam2;
+    DBuf<double4> lamT2;
+    DBuf<unsigned char> flag2;
+    DBuf<pu4> lines, red;
+    DBuf<unsigned> arrive;  // [PT_MAX_PARTS] check-ins, then the decision
+    unsigned seq = 0, epoch = 0;
+    bool global = false;    // a part may have more bodies than LDS slots
+    bool everOver = false;  // one had, unexpectedly
+    PartList Q{};
+    void release() {
+      mask.release(); listStart.release(); list.release(); nxt.release();
+      grid.release(); hist.release(); cellStart.release(); partOf.release();
+      partCnt.release(); partIds.release(); bktCnt.release(); bkt.release(); ent.release();
+      rank.release(); lam2.release(); lamT2.release(); flag2.release(); lines.release();
+      red.release(); arrive.release();
+    }
+  };
+  PartJob partsV, partsP;
+  static constexpr long PT_SINGLE = 4;
+  static constexpr size_t PT_LINE_BYTES_MAX = 0xFFFFFF00u;  // (32-bit line offsets)
+  // The partitioned loop takes rows whose classes leave out the last one (62, whose rows may share
+  // a body), up to maxRows of them.
+  bool partsTake(int rows, int numColors, int nd, long maxRows) const {
+    return partRows > 0 && blockRows > 0 && partsBusy == 0 && numColors <= PT_COLORS &&
+           rows <= maxRows && (size_t)rows * 4 * 16 * nd <= PT_LINE_BYTES_MAX;
+  }
+  // Velocity rows: above this many the launches per colour move their rows faster than 224
+  // workgroups whose bodies no longer all fit in LDS (ms per substep, launches / partition: 0.55M
+  // rows of a 1M pour 6.79 / 6.28, 1.96M rows of a resting 1M bed 16.0 / 17.0).
+  static constexpr long PARTS_V_ROWS = 1L << 20;
+  static int partLevels(int parts) {  // about 64 cells per part
+    int l = 6;
+    while ((1 << l) < 64 * parts && (1 << l) < PT_MAX_CELLS) ++l;
+    return l;
+  }
+  // partition `rows` rows with bodies ends[] (ids below `ids`, at pos[]) in the classes cs
+  template <bool VEL>
+  void buildParts(PartJob& J, const int2* ends, const double4* posOf, int ids, int rows,
+                  const ClassStarts& cs, int numColors, int cap) {
+    // Up to partRows x PT_SINGLE rows one workgroup holds a colour's rows at once and no states
+    // travel (300 spheres, 570 + 1,010 rows: 0.49 ms per substep in one workgroup, 0.66 in
+    // several); beyond, a chunk of each colour per workgroup is best (9,001 spheres at 160 / 256 /
+    // 384 / 640 rows per workgroup: 1.12 / 1.09 / 1.15 / 1.30 ms).
+    const int parts = rows <= PT_SINGLE * partRows
+                          ? 1
+                          : (int)std::min<long>(std::min(partMax, PT_MAX_PARTS),
+                                                (rows + partRows - 1) / partRows);
+    const int levels = partLevels(parts), cells = parts > 1 ? 1 << levels : 0;
+    const long most = std::min<long>(ids, 2L * rows);
+    // (a part's bodies number at most about 1.7 times the average: k_part_hist's weights)
+    const long room = 2 * ((most + parts - 1) / parts) + 64;
+    const int capL = (int)std::min<long>(cap, room);
+    J.global = room > cap || J.everOver;
+    const int bkts = parts * std::max(1, numColors);
+    J.partOf.ensure(ids + 1, st);
+    J.partCnt.ensure(PT_MAX_PARTS + 1, st);  // (and the lists' counter)
+    J.partIds.ensure((size_t)parts * capL, st);
+    J.bktCnt.ensure(2 * bkts, st);
+    J.bkt.ensure(bkts, st);
+    const long entries = (parts > 1 ? 2L : 1L) * rows + (long)PT_CHUNK * bkts;
+    J.ent.ensure(entries, st);
+    J.nxt.ensure(entries, st);
+    if (parts > 1) {
+      J.grid.ensure(1, st);
+      J.mask.ensure(ids + 1, st);
+      J.listStart.ensure(ids + 1, st);
+      J.list.ensure(2L * rows + 1, st);
+      J.hist.ensure(PT_MAX_CELLS + 1, st);
+      J.cellStart.ensure(PT_MAX_CELLS + 1, st);
+      J.rank.ensure(rows + 1, st);
+    }
+    J.red.ensure(2 * PT_MAX_PARTS, st);
+    J.arrive.ensure(PT_MAX_PARTS + 1, st);
+    if (VEL && parts > 1) {
+      J.lam2.ensure(rows, st);
+      J.lamT2.ensure(rows, st);
+      J.flag2.ensure(rows, st);
+    }
+    if (parts > 1) J.lines.ensure((size_t)rows * 4 * (VEL ? 6 : 3), st);
+    PartList& Q = J.Q;
+    Q = PartList{parts, numColors, capL, J.grid.p, J.mask.p, J.listStart.p, J.list.p,
+                 J.partCnt.p + PT_MAX_PARTS, J.hist.p, J.cellStart.p, J.partOf.p, J.partCnt.p,
+                 J.partIds.p, J.bktCnt.p, J.bkt.p, J.rank.p, J.ent.p, J.nxt.p, J.lam2.p,
+                 J.lamT2.p, J.flag2.p};
+    if (parts > 1) {  // (a loop of one workgroup builds its partition itself)
+      k_part_begin<<<nblk(std::max(std::max(ids, cells), 2 * bkts)), TPB, 0, st>>>(
+          Q, gridD.p, ids, cells, levels);
+      k_part_colours<<<nblk(rows), TPB, 0, st>>>(Q, ends, cs, rows);
+      k_part_hist<<<nblk(ids), TPB, 0, st>>>(Q, posOf, ids);
+      scanQuiet(J.hist.p, J.cellStart.p, cells);
+      k_part_assign<<<(ids + 1023) / 1024, 1024, 0, st>>>(Q, posOf, ids, cells);
+      k_part_count<<<(rows + 1023) / 1024, 1024, 0, st>>>(Q, ends, cs, rows);
+      k_part_ranges<<<1, 1024, 0, st>>>(Q);
+      k_part_fill<VEL><<<nblk(rows), TPB, 0, st>>>(dD, Q, ends, cs, rows);
+    }
+    HIPCHECK(hipGetLastError());
+  }
+  // the exchange areas for a launch of at most `passes` passes
+  PartSync partSync(PartJob& J, int rows, int nd, long passes, bool refuse) {
+    PartSync Y{};
+    if (J.seq > 0xFFFFFFFFu - (unsigned long)passes - 2 || J.epoch >= 0x7FFFFFFEu) {
+      // the numbers start over: no line may hold an old one
+      zero(J.lines.p, J.lines.cap);
+      zero(J.red.p, J.red.cap);
+      zero(J.arrive.p, J.arrive.cap);
+      J.seq = J.epoch = 0;
+    }
+    Y.lines = J.lines.p;
+    Y.half = (unsigned)((size_t)rows * 2 * 16 * nd);
+    Y.lineBytes = 2 * Y.half;
+    Y.red = J.red.p;
+    Y.arrive = J.arrive.p;
+    Y.decision = J.arrive.p + PT_MAX_PARTS;
+    Y.seq0 = J.seq;
+    J.seq += (unsigned)passes + 1;
+    Y.epoch = ++J.epoch;
+    Y.busy = ctl.p + CTL_PARTS_BUSY;
+    Y.over = ctl.p + CTL_PARTS_OVER;
+    Y.fail = ctl.p + CTL_PARTS_FAIL;
+    Y.refuse = refuse ? 1 : 0;
+    return Y;
   }
   bool vFusedRec = false;  // the timed K_VBLOCK record covers both loops of the stage
   long vBlockRec[2] = {-1, -1}, pBlockRec = -1;
@@ -1865,7 +2014,7 @@ struct pd_sim {
   void tagSweepRec(long rec) {
     if (rec >= 0 && curSweepTag >= 0) sweepRecs.push_back({rec, curSweepTag});
   }
-  int posSweepsPrev = 1;  // sweeps of the last batched position loop (first batch size)
+  int posSweepsPrev = 1;  // sweeps of the last position loop
   // contact lists of at least this many contacts start their colouring before the velocity stage
   static constexpr int EARLY_CONTACT_COLOURING = 1 << 18;
   // The contact colouring's last class (62) may hold rows sharing a body (shell shapes: the many
@@ -2160,8 +2309,8 @@ struct pd_sim {
     const bool hostLoop = velLeftover > 0 || (usePGS && stabMode >= 2) || !useGS ||
                           legacyFriction;
     const bool smallV = nRowsV <= blockRows;
-    // the whole velocity stage in one launch on LDS-staged bodies
-    const bool fusedV = !hostLoop && smallV && velIters > 0 && ldsLoop && nRowsV <= VL_ROWS;
+    // the whole velocity stage in one launch over a partition of the bodies
+    const bool fusedV = !hostLoop && velIters > 0 && ldsLoop && partsTake(nRowsV, numColors, 6, PARTS_V_ROWS);
     const size_t R = nRowsV + 1;
     vAB.ensure(R, st); vN.ensure(R, st); vTA.ensure(R, st); vTB.ensure(R, st); vRA.ensure(R, st);
     vRB.ensure(R, st); vVt0.ensure(R, st); vLamT.ensure(R, st); vVn0.ensure(R, st);
@@ -2217,14 +2366,13 @@ struct pd_sim {
     mark(ST_VSWEEP);
     if (fusedV) {
       // warm start, sweep loop, stabilization gate, side flags and stabilization loop in one
-      // launch on bodies staged in LDS; above ldsKeys / 2 rows staging may give up, and the
-      // same sequence of global-memory launches follows, gated on its flag
-      const double stopThr = usePGS ? 0.02 * vRest : vRest;
+      // launch
+      const ClassStarts cs = classStarts(vs);
       VStage S{};
       S.warm = usePGS ? 1 : 0;
       S.iters = velIters;
       S.thr = vRest;
-      S.stopThr = stopThr;
+      S.stopThr = usePGS ? 0.02 * vRest : vRest;
       S.stop = ctl.p + CTL_STOP_V;
       S.count = ctl.p + CTL_SWEEPS_V;
       S.gate = usePGS ? 1 : 0;
@@ -2237,30 +2385,15 @@ struct pd_sim {
       S.gHat = gHat;
       S.riseThr = 8.0 * dt * gMagP;
       S.approachThr = 8.0 * dt * gMagP;
-      int* fb = ctl.p + CTL_VFALLBACK;
+      const int cap = ldsBodies < LDS_BODIES_MAX ? ldsBodies : PT_VBODIES;
+      buildParts<true>(partsV, vAB.p, posPred.p, numReal, nRowsV, cs, numColors, cap);
+      const PartSync Y = partSync(partsV, nRowsV, 6, 3L * velIters + 4,
+                                  ldsKeys < LDS_KEYS_MAX && 2L * nRowsV > ldsKeys);
+      const PartList& Q = partsV.Q;
       kernBegin();
-      if (usePGS)
-        k_vsolve_lds<1><<<1, VBLOCK_THREADS, 0, st>>>(dD, P, classStarts(vs), numColors, nm, S, fb,
-                                                       ldsBodies, ldsKeys);
-      else
-        k_vsolve_lds<2><<<1, VBLOCK_THREADS, 0, st>>>(dD, P, classStarts(vs), numColors, nm, S, fb,
-                                                       ldsBodies, ldsKeys);
-      if (2 * (long)nRowsV > ldsKeys) {
-        if (usePGS)
-          vLoop(0, P, vs, numColors, 1, 0.0, 0.0, ctl.p + CTL_NONE, ctl.p + CTL_NONE, nullptr, fb);
-        vLoop(usePGS ? 1 : 2, P, vs, numColors, velIters, vRest, stopThr, ctl.p + CTL_STOP_V,
-              ctl.p + CTL_SWEEPS_V, nullptr, fb);
-        if (usePGS) {
-          k_stab_gate<<<1, 1, 0, st>>>(bits.p + 1, ctl.p, stabMode, vRestS, fb);
-          if (stabMode == 1) {
-            if (nRowsV > 0)
-              k_side_flags<<<nblk(nRowsV), TPB, 0, st>>>(dD, nRowsV, gHat, S.riseThr,
-                                                         S.approachThr, ctl.p + CTL_STAB_RUN, fb);
-            vLoop(1, P, vs, numColors, 2 * velIters, vRestS, vRestS, ctl.p + CTL_STOP_S,
-                  ctl.p + CTL_SWEEPS_S, ctl.p + CTL_STAB_RUN, fb);
-          }
-        }
-      }
+      auto* const kernel = usePGS ? (partsV.global ? &k_vsolve_lds<1, true> : &k_vsolve_lds<1, false>)
+                                  : (partsV.global ? &k_vsolve_lds<2, true> : &k_vsolve_lds<2, false>);
+      kernel<<<Q.numParts, PT_THREADS, Q.cap * 48, st>>>(dD, P, cs, S, Q, Y);
       vBlockRec[0] = kernEnd(K_VBLOCK, nRowsV);
       vFusedRec = true;
       HIPCHECK(hipGetLastError());
@@ -2284,14 +2417,13 @@ struct pd_sim {
       });
       mark(ST_STAB);
       if (usePGS) {
-        k_stab_gate<<<1, 1, 0, st>>>(bits.p + 1, ctl.p, stabMode, vRestS, nullptr);
+        k_stab_gate<<<1, 1, 0, st>>>(bits.p + 1, ctl.p, stabMode, vRestS);
         if (smallV) {
           // the gate stays on the device: the flags kernel and the loop read it
           if (stabMode == 1 && velIters > 0) {
             if (nRowsV > 0)
               k_side_flags<<<nblk(nRowsV), TPB, 0, st>>>(dD, nRowsV, gHat, 8.0 * dt * gMagP,
-                                                         8.0 * dt * gMagP, ctl.p + CTL_STAB_RUN,
-                                                         nullptr);
+                                                         8.0 * dt * gMagP, ctl.p + CTL_STAB_RUN);
             kernBegin();
             vLoop(1, P, vs, numColors, 2 * velIters, vRestS, vRestS, ctl.p + CTL_STOP_S,
                   ctl.p + CTL_SWEEPS_S, ctl.p + CTL_STAB_RUN);
@@ -2301,7 +2433,7 @@ struct pd_sim {
           if (nRowsV > 0)
             k_side_flags<<<nblk(nRowsV), TPB, 0, st>>>(dD, nRowsV, gHat, 8.0 * dt * gMagP,
                                                        8.0 * dt * gMagP, ctl.p + CTL_STAB_RUN,
-                                                       nullptr, vbActive);
+                                                       vbActive);
           sweepLoop(2 * velIters, ctl.p + CTL_STOP_S, [&, ss = 0]() mutable {
             if (ss == 0) k_sweep_begin<<<1, 1, 0, st>>>(bits.p + 1, ctl.p + CTL_STOP_S);
             curSweepTag = 4096 + ss++;
@@ -2348,8 +2480,7 @@ struct pd_sim {
           writeN(ctl.p + CTL_STAB_RUN, &one, 1);
           if (stabMode == 1 && nRowsV > 0)
             k_side_flags<<<nblk(nRowsV), TPB, 0, st>>>(dD, nRowsV, gHat, 8.0 * dt * gMagP,
-                                                       8.0 * dt * gMagP, ctl.p + CTL_STAB_RUN,
-                                                       nullptr);
+                                                       8.0 * dt * gMagP, ctl.p + CTL_STAB_RUN);
           if (stabMode == 4) {
             orderedStabilization(gHat, vRestS);
           } else if (stabMode == 2) {
@@ -2440,7 +2571,11 @@ struct pd_sim {
     pLam.ensure(nRowsP + 1, st);
     refreshDev();
     // with the batched position loop ahead, the rows launch also clears its residual
-    const bool posBatches = useGS && posLeftover == 0 && nRowsP > blockRows;
+    // (a loop that stops after a sweep or two does not repay building a partition)
+    const bool posParts = useGS && posLeftover == 0 && posIters > 0 && nRowsP > 0 &&
+                          (posSweepsPrev > 2 || nRowsP > blockRows) &&
+                          partsTake(nRowsP, numPosColors, 3, 1L << 30);
+    const bool posBatches = useGS && posLeftover == 0 && nRowsP > blockRows && !posParts;
     if (nRowsP > 0)
       k_prows<<<nblk(nc), TPB, 0, st>>>(dD, nc, posBatches ? bits.p : nullptr);
     mark(ST_PSWEEP);
@@ -2455,10 +2590,22 @@ struct pd_sim {
         stats.sweeps_pos++;
       }
       HIPCHECK(hipGetLastError());
+    } else if (posParts) {
+      const ClassStarts pcs = classStarts(ps);
+      buildParts<false>(partsP, pAB.p, posPred.p, numParticles, nRowsP, pcs, numPosColors,
+                        PT_PBODIES);
+      const PartSync Y = partSync(partsP, nRowsP, 3, posIters + 1L, false);
+      const PartList& Q = partsP.Q;
+      kernBegin();
+      auto* const kernel = partsP.global ? &k_psolve_lds<true> : &k_psolve_lds<false>;
+      kernel<<<Q.numParts, PT_THREADS, Q.cap * 24, st>>>(
+          dD, pcs, posIters, posTol, ctl.p + CTL_STOP_P, ctl.p + CTL_SWEEPS_P, Q, Y);
+      pBlockRec = kernEnd(K_PBLOCK, nRowsP);
+      HIPCHECK(hipGetLastError());
     } else if (posLeftover == 0 && nRowsP <= blockRows) {
       if (posIters > 0) {
         kernBegin();
-        k_psolve_block<<<1, BLOCK_SOLVER_THREADS, 0, st>>>(dD, classStarts(ps), numPosColors, nc,
+        k_psolve_block<<<1, BLOCK_SOLVER_THREADS, 0, st>>>(dD, classStarts(ps), numPosColors,
                                                            posIters, posTol, ctl.p + CTL_STOP_P,
                                                            ctl.p + CTL_SWEEPS_P);
         pBlockRec = kernEnd(K_PBLOCK, nRowsP);
@@ -2537,7 +2684,6 @@ struct pd_sim {
         if (finalCtl[CTL_STOP_P]) break;
         batch *= 2;
       }
-      posSweepsPrev = finalCtl[CTL_SWEEPS_P];
     } else {
       // colouring leftovers: the coloured sweep, then Jacobi over the uncoloured contacts
       if (posIters > 0) buildIncidence<1>(nc, 1);
@@ -2574,7 +2720,19 @@ struct pd_sim {
         stats.sweeps_stab = c[CTL_SWEEPS_S];
         stats.stab_ran = usePGS ? c[CTL_STAB_RUN] : 0;
       }
-      if (useGS && posLeftover == 0) stats.sweeps_pos = c[CTL_SWEEPS_P];
+      if (useGS && posLeftover == 0) posSweepsPrev = stats.sweeps_pos = c[CTL_SWEEPS_P];
+      if (c[CTL_PARTS_FAIL])
+        throw std::runtime_error("sweep loop: a workgroup waited too long for another");
+      // a partitioned loop that found the device busy ran in one workgroup, slowly: the launches
+      // per colour take over for a while, longer each time
+      if (partsBusy > 0) {
+        --partsBusy;
+      } else if (c[CTL_PARTS_OVER]) {
+        partsV.everOver = partsP.everOver = true;
+      } else if (c[CTL_PARTS_BUSY] && ldsKeys == LDS_KEYS_MAX) {
+        partsBusy = partsBusyNext;
+        partsBusyNext = std::min(4096L, 2 * partsBusyNext);
+      }
       maxOverlap = bitsd(b2[0]);
       maxApproach = bitsd(b2[1]);
     }
@@ -3891,13 +4049,20 @@ int pd_set_tuning(pd_sim* s, const char* name, long value) {
       if (value != 0 && value != 1) throw ArgError("velocity_loop_lds must be 0 or 1");
       s->ldsLoop = value != 0;
     } else if (k == "velocity_loop_lds_bodies") {
-      if (value < 1 || value > VL_BODIES)
-        throw ArgError("velocity_loop_lds_bodies must be in [1, " + std::to_string(VL_BODIES) + "]");
+      if (value < 1 || value > pd_sim::LDS_BODIES_MAX)
+        throw ArgError("velocity_loop_lds_bodies must be in [1, " + std::to_string(pd_sim::LDS_BODIES_MAX) + "]");
       s->ldsBodies = (int)value;
     } else if (k == "velocity_loop_lds_keys") {
-      if (value < 1 || value > VL_KEYS)
-        throw ArgError("velocity_loop_lds_keys must be in [1, " + std::to_string(VL_KEYS) + "]");
+      if (value < 1 || value > pd_sim::LDS_KEYS_MAX)
+        throw ArgError("velocity_loop_lds_keys must be in [1, " + std::to_string(pd_sim::LDS_KEYS_MAX) + "]");
       s->ldsKeys = (int)value;
+    } else if (k == "partition_rows") {
+      if (value < 0) throw ArgError("partition_rows must be >= 0");
+      s->partRows = value;
+    } else if (k == "partition_workgroups") {
+      if (value < 1 || value > PT_MAX_PARTS)
+        throw ArgError("partition_workgroups must be in [1, " + std::to_string(PT_MAX_PARTS) + "]");
+      s->partMax = (int)value;
     } else if (k == "candidate_skin_permille") {
       if (value < 0) throw ArgError("candidate_skin_permille must be >= 0");
       s->candSkinFrac = std::min<long>(value, 100000) / 1000.0;
@@ -3972,7 +4137,7 @@ int pd_get_stats_log(pd_sim* s, pd_stats* out, int cap) {
 const char* pd_kernel_name(int k) {
   static const char* names[pd_sim::K_COUNT] = {
       "k_vsweep",  "k_psweep",      "k_bp_query",     "k_np_pairs",
-      "k_predict", "k_reintegrate", "k_vsolve_lds", "k_psolve_block"};
+      "k_predict", "k_reintegrate", "k_vsolve_lds", "k_psolve_block"};  // (the one-launch position loops)
   return (k >= 0 && k < pd_sim::K_COUNT) ? names[k] : "";
 }
 const char* pd_stage_name(int stage) {

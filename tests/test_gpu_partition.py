@@ -1,0 +1,73 @@
+"""The sweep loops over a spatial partition of the bodies (pd_parts.hpp) against the CPU oracle:
+every substep's state, counters and ledger, at partitions from one workgroup to one row per few."""
+import numpy as np
+import pytest
+
+from test_gpu_parity import run_pair
+
+# rows per workgroup: one workgroup for all rows, a few, and many of a chunk (32 rows) or less
+ROWS = [100000, 200, 33, 9]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["bed", "bed_periodic", "gas", "bed_walls"])
+@pytest.mark.parametrize("rows", ROWS)
+def test_partition_sizes(hip_lib, kind, rows):
+    run_pair(kind, 500, 12, tuning={"partition_rows": rows})
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,n,steps", [("column_small_box", 64, 8), ("boxes", 48, 8),
+                                          ("cylinders", 48, 8), ("bed_small_box", 60, 8),
+                                          ("big_among_small", 4000, 3)])
+@pytest.mark.parametrize("rows", [200, 9])
+def test_partition_shapes_and_twins(hip_lib, kind, n, steps, rows):
+    # several points per manifold, every sphere with images of its neighbours, and (the big sphere)
+    # colourings whose last class keeps the loops off the partition
+    run_pair(kind, n, steps, tuning={"partition_rows": rows})
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["bed", "bed_periodic", "gas"])
+@pytest.mark.parametrize("tuning", [{"velocity_loop_lds_bodies": 3}, {"velocity_loop_lds_keys": 16},
+                                    {"partition_workgroups": 2}],
+                         ids=["lds-and-global", "refused-check-in", "two-workgroups"])
+def test_partition_storage_and_check_in(hip_lib, kind, tuning):
+    # parts with more bodies than LDS slots; workgroups that agree to leave at the check-in, so that
+    # one of them runs the loop; more rows per workgroup than asked for
+    run_pair(kind, 300, 10, tuning={"partition_rows": 20, **tuning})
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("over", [{"material": (0.3, 0.0, 0.5)}, {"material": (0.6, 0.4, 0.0)},
+                                  {"stab": "off"}, {"iters": (1, 1)}, {"iters": (0, 3)}],
+                         ids=["no-tangential", "frictionless", "no-stabilization", "one-sweep",
+                              "no-position-loop"])
+def test_partition_options(hip_lib, over):
+    run_pair("bed_periodic", 400, 10, tuning={"partition_rows": 60}, **over)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,n,tunings", [
+    # enough rows for more than a hundred workgroups of several chunks per colour
+    ("bed_periodic", 20000, [{}, {"partition_workgroups": 7}]),
+    # a sphere wider than its box: rows of a body and its own image
+    ("big_among_small", 300, [{}, {"partition_rows": 10}])])
+def test_partition_equals_the_launches_per_colour(hip_lib, kind, n, tunings):
+    from peclet.dem import Simulation
+    from scenes import apply_scene, make_scene
+
+    scene = make_scene(kind, n, 5)
+    runs = []
+    for tuning in [{"block_solver_rows": 0}] + tunings:
+        print(tuning, flush=True)
+        h = apply_scene(Simulation(n), scene)
+        for key, value in tuning.items():
+            h.set_tuning(key, value)
+        h.step_n(scene["dt"], 6)
+        runs.append((h.get_positions(), h.get_velocities(), h.get_angular_velocities(),
+                     *h.debug_ledger(), h.get_stats()))
+        h.close()
+    for other in runs[1:]:
+        for a, b in zip(runs[0], other):
+            assert np.array_equal(a, b) if isinstance(a, np.ndarray) else a == b
