@@ -2909,7 +2909,7 @@ __global__ void k_side_flags(const Dev* __restrict__ Dp, int numRows, d3 gHat, d
 // ---- device-side loop control: ctl[0..] ints (see pd_sim.hip), sweeps after a stop are no-ops
 enum { CTL_STOP_V = 0, CTL_SWEEPS_V, CTL_STAB_RUN, CTL_STOP_S, CTL_SWEEPS_S, CTL_STOP_P,
        CTL_SWEEPS_P, CTL_NONE, CTL_PARTS_BUSY, CTL_PARTS_OVER,
-       CTL_PARTS_FAIL, CTL_COUNT };
+       CTL_PARTS_FAIL, CTL_DUMP, CTL_COUNT };
 __global__ void k_sweep_begin(unsigned long long* bits, const int* stop) {
   if (!*stop) *bits = 0ull;
 }

@@ -48,8 +48,8 @@ namespace pd {
 
 typedef unsigned pu4 __attribute__((ext_vector_type(4)));
 
-constexpr int PT_THREADS = 512;
-constexpr int PT_WAVES = PT_THREADS / 64;
+constexpr int PT_V_THREADS = 512;   // (a velocity row's ~215 VGPRs allow two waves per SIMD)
+constexpr int PT_P_THREADS = 1024;  // (a position row's ~85 four)
 constexpr int PT_CHUNK = 32;  // rows of a chunk: two lanes each
 constexpr int PT_MAX_PARTS = 256;
 constexpr int PT_COLORS = 62;  // the last class (62) may hold rows sharing a body: not taken here
@@ -59,8 +59,11 @@ constexpr int PT_REMOTE = 0xFFFD;  // another part's body: received
 constexpr int PT_GLOBAL = 0xFFFE;  // this part's body without an LDS slot: in global memory
 constexpr int PT_NONE = 0xFFFF;    // no body (plane or wall)
 // LDS bodies per part: the states fill at most 150 KB of the 160 KB
+constexpr int PT_LDS_BYTES = 158 * 1024;
 constexpr int PT_VBODIES = 3200;  // 48 B each
 constexpr int PT_PBODIES = 6400;  // 24 B each
+// dynamic LDS of a loop: bodies, then 16 bytes per class
+inline int partLdsBytes(int cap, int classes, int nd) { return ((cap * nd * 8 + 15) & ~15) + 16 * classes; }
 
 // cells of the partition: a box halved PT levels times, always across its longest edge; the
 // cell index is the path of halves, so consecutive cells are close in space
@@ -461,40 +464,29 @@ __device__ __forceinline__ unsigned long long partMax(unsigned long long m, cons
 }
 
 // ---- the pass over a part's rows -----------------------------------------------------------
-// A part's chunks in colour order; chunk j of colour c belongs to wave (base[c] + j) mod PT_WAVES.
-struct PartChunks {
-  int first[PT_COLORS], between[PT_COLORS], count[PT_COLORS], base[PT_COLORS + 1];
-};
-__device__ __forceinline__ void chunksLoad(const PartList& Q, int me, PartChunks& ch) {
-  for (int c = threadIdx.x; c < Q.numColors; c += blockDim.x) {
-    const int4 b = Q.bkt[me * Q.numColors + c];
-    ch.first[c] = b.x;
-    ch.between[c] = b.y;
-    ch.count[c] = b.z;
+// A part's chunks in class order: class c has table[c] = (first entry, entries between parts,
+// entries, base), and its chunk j belongs to wave (base + j) mod WAVES.
+template <int WAVES>
+__device__ __forceinline__ void tableLoad(const PartList& Q, int me, int4* table) {
+  if (Q.numParts > 1) {
+    for (int c = threadIdx.x; c < Q.numColors; c += blockDim.x) table[c] = Q.bkt[me * Q.numColors + c];
+    __syncthreads();
   }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int b = 0;
-    for (int c = 0; c < Q.numColors; ++c) {
-      ch.base[c] = b;
-      b = (b + (ch.count[c] + PT_CHUNK - 1) / PT_CHUNK) % PT_WAVES;
+  if (threadIdx.x < 64) {
+    int at = 0;
+    for (int c0 = 0; c0 < Q.numColors; c0 += 64) {
+      const int c = c0 + (int)threadIdx.x;
+      const int n = c < Q.numColors ? (table[c].z + PT_CHUNK - 1) / PT_CHUNK : 0;
+      int inc = n;
+      for (int off = 1; off < 64; off <<= 1) {
+        const int x = __shfl_up(inc, off, 64);
+        if ((int)threadIdx.x >= off) inc += x;
+      }
+      if (c < Q.numColors) table[c].w = (at + inc - n) % WAVES;
+      at += __shfl(inc, 63, 64);
     }
   }
   __syncthreads();
-}
-__device__ __forceinline__ int chunkFirst(const PartChunks& ch, int c, int wave) {
-  const int j = wave - ch.base[c];
-  return j < 0 ? j + PT_WAVES : j;
-}
-// the wave's next chunk in the cycle of colours (c = -1: the wave has none)
-__device__ __forceinline__ void chunkNext(const PartChunks& ch, int numColors, int wave, int& c,
-                                          int& j) {
-  for (int t = 0; t <= numColors; ++t) {
-    if (j * PT_CHUNK < ch.count[c]) return;
-    c = c + 1 == numColors ? 0 : c + 1;
-    j = chunkFirst(ch, c, wave);
-  }
-  c = -1;
 }
 // Workgroup barrier that orders LDS only.  __syncthreads also waits for every global access in
 // flight: the acknowledgements of the impulse stores and the loads issued ahead.
@@ -536,7 +528,7 @@ struct ChunkAt {
 };
 template <class R, bool GLOB>
 struct PartRun {
-  static constexpr int ND = R::ND;
+  static constexpr int ND = R::ND, WAVES = R::THREADS / 64;
   // (by value: references to kernel arguments kept in an object would place the arguments in
   // scratch memory)
   const R rows;
@@ -545,8 +537,8 @@ struct PartRun {
   const int* const nxt;  // [entries][2]
   int* const fail;
   const unsigned half;
-  const PartChunks& ch;
-  double* const body;  // LDS [cap][ND]
+  const int4* const table;  // LDS [numColors]
+  double* const body;       // LDS [cap][ND]
   const __amdgpu_buffer_rsrc_t lines;
   unsigned pass;  // number of the current pass
   int wave, sub;
@@ -559,23 +551,40 @@ struct PartRun {
   typename R::Row cur;
 
   __device__ __forceinline__ PartRun(const R& r, const PartList& q, const PartSync& y,
-                                     const PartChunks& c, double* b)
-      : rows(r), numColors(q.numColors), ent(q.ent), nxt((const int*)q.nxt), fail(y.fail), half(y.half), ch(c), body(b),
+                                     const int4* t, double* b)
+      : rows(r), numColors(q.numColors), ent(q.ent), nxt((const int*)q.nxt), fail(y.fail), half(y.half), table(t), body(b),
         lines(lineRsrc(y.lines, y.lineBytes)), pass(y.seq0) {
     wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     sub = (int)(threadIdx.x & 63) >> 1;
     isB = threadIdx.x & 1;
     start();
   }
-  __device__ __forceinline__ ChunkAt after(ChunkAt a) const {
-    a.j += PT_WAVES;
-    chunkNext(ch, numColors, wave, a.c, a.j);
+  // the wave's first chunk of a class
+  __device__ __forceinline__ int firstChunk(int base) const {
+    const int j = wave - base;
+    return j < 0 ? j + WAVES : j;
+  }
+  // the wave's chunk at or after a in the cycle of classes (c = -1: the wave has none)
+  __device__ __forceinline__ ChunkAt chunkAt(ChunkAt a) const {
+    int4 t = table[a.c];
+    for (int n = 0; n <= numColors; ++n) {
+      if (a.j * PT_CHUNK < t.z) return a;
+      a.c = a.c + 1 == numColors ? 0 : a.c + 1;
+      t = table[a.c];
+      a.j = firstChunk(t.w);
+    }
+    a.c = -1;
     return a;
+  }
+  __device__ __forceinline__ ChunkAt after(ChunkAt a) const {
+    a.j += WAVES;
+    return chunkAt(a);
   }
   // Loads ahead have no condition (a lane past the chunk's end takes the last entry): a value that
   // may or may not be loaded is settled, and waited for, where the condition ends.
   __device__ __forceinline__ void entry(ChunkAt a, int& k, int& l, int& ia, int& ib, int& n) const {
-    const int at = ch.first[a.c] + min(a.j * PT_CHUNK + sub, ch.count[a.c] - 1);
+    const int4 t = table[a.c];
+    const int at = t.x + min(a.j * PT_CHUNK + sub, t.z - 1);
     const int4 e = ent[at];
     n = nxt[2 * at + (isB ? 1 : 0)];
     k = e.x;
@@ -589,8 +598,7 @@ struct PartRun {
     finished = true;
     pending = false;
     if (numColors == 0) return;
-    at0 = ChunkAt{0, chunkFirst(ch, 0, wave)};
-    chunkNext(ch, numColors, wave, at0.c, at0.j);
+    at0 = chunkAt(ChunkAt{0, firstChunk(table[0].w)});
     if (at0.c < 0) return;
     at1 = after(at0);
     entry(at0, ek, el, ea, eb, en);
@@ -656,12 +664,12 @@ struct PartRun {
   // that are their body's first row in a pass (what the rows before do not send)
   __device__ __forceinline__ void sendRows(unsigned seq, bool all) const {
     for (int c = 0; c < numColors; ++c) {
-      const int nbt = ch.between[c];
-      for (int j = chunkFirst(ch, c, wave); j * PT_CHUNK < nbt; j += PT_WAVES) {
+      const int4 t = table[c];
+      for (int j = firstChunk(t.w); j * PT_CHUNK < t.y; j += WAVES) {
         const int at = j * PT_CHUNK + sub;
-        if (at >= nbt) continue;
-        const int4 o = ent[ch.first[c] + at];
-        const int loc = own(o.y), first = nxt[2 * (ch.first[c] + at) + (isB ? 1 : 0)] & 1;
+        if (at >= t.y) continue;
+        const int4 o = ent[t.x + at];
+        const int loc = own(o.y), first = nxt[2 * (t.x + at) + (isB ? 1 : 0)] & 1;
         if (loc == PT_REMOTE || !(all || first)) continue;
         double x[ND];
         bodyLoad(loc, isB ? o.w : o.z, x);
@@ -684,13 +692,16 @@ struct PartRun {
   __device__ __forceinline__ unsigned long long sweep(double thr) {
     ++pass;
     unsigned long long m = 0;
+    int4 tn = numColors > 0 ? table[0] : make_int4(0, 0, 0, 0);
     for (int c = 0; c < numColors; ++c) {
-      const int n = ch.count[c];
+      const int4 t = tn;
+      tn = table[c + 1 < numColors ? c + 1 : 0];
+      const int n = t.z;
       if (n == 0) continue;
       // the earlier colours' states are in LDS (or in global memory)
       if (GLOB) __syncthreads();
       else ldsBarrier();
-      int j = chunkFirst(ch, c, wave);
+      int j = firstChunk(t.w);
       if (j * PT_CHUNK >= n) {  // nothing to do in this colour: get ready for the next one
         if (pending) advance();
         else finish();
@@ -718,7 +729,7 @@ struct PartRun {
           const unsigned long long a = dbits(amax);
           m = a > m ? a : m;
         }
-        j += PT_WAVES;
+        j += WAVES;
         if (j * PT_CHUNK >= n) break;
         advance();
       }
@@ -732,7 +743,7 @@ struct PartRun {
 // (v, w).  The odd lane works with the normal, the friction impulse and every relative quantity
 // negated, which changes no rounding: what it adds to body B is what the row adds to it.
 struct VelPart {
-  static constexpr int ND = 6;
+  static constexpr int ND = 6, THREADS = PT_V_THREADS;
   struct Row {
     d3 N, r, Tau;  // normal sum and this lane's arm and angular row
     double rest, mu, sgn, vn0, lenN, invLenN;
@@ -991,17 +1002,26 @@ struct VStage {
   double riseThr, approachThr;
 };
 // The whole partition of a loop that one workgroup runs, built by that workgroup: a body's first
-// row gives it its place, and the entries are the classes' rows as they lie.
+// row gives it its place, and the entries are the classes' rows as they lie.  table: LDS, one int4
+// per class.
 __device__ __forceinline__ void partSingle(const PartList& Q, const PD_G int2* ends,
-                                           const ClassStarts& cs, int* first) {
+                                           const ClassStarts& cs, int4* table) {
   __shared__ int bodies;
   const int r0 = cs.s[0], r1 = cs.s[Q.numColors];
-  if (threadIdx.x == 0) {
-    bodies = 0;
+  if (threadIdx.x == 0) bodies = 0;
+  if (threadIdx.x < 64) {
     int at = 0;
-    for (int c = 0; c < Q.numColors; ++c) {
-      first[c] = at;
-      at += (cs.s[c + 1] - cs.s[c] + PT_CHUNK - 1) & ~(PT_CHUNK - 1);
+    for (int c0 = 0; c0 < Q.numColors; c0 += 64) {
+      const int c = c0 + (int)threadIdx.x;
+      const int n = c < Q.numColors ? cs.s[c + 1] - cs.s[c] : 0;
+      const int padded = (n + PT_CHUNK - 1) & ~(PT_CHUNK - 1);
+      int inc = padded;
+      for (int off = 1; off < 64; off <<= 1) {
+        const int x = __shfl_up(inc, off, 64);
+        if ((int)threadIdx.x >= off) inc += x;
+      }
+      if (c < Q.numColors) table[c] = make_int4(at + inc - padded, 0, n, 0);
+      at += __shfl(inc, 63, 64);
     }
   }
   for (int k = r0 + (int)threadIdx.x; k < r1; k += blockDim.x) {
@@ -1011,7 +1031,7 @@ __device__ __forceinline__ void partSingle(const PartList& Q, const PD_G int2* e
   }
   __syncthreads();
   auto place = [&](int id) {
-    if (atomicCAS(&Q.partOf[id], -1, -2) != -1) return;
+    if (ldDevice(&Q.partOf[id]) != -1 || atomicCAS(&Q.partOf[id], -1, -2) != -1) return;
     const int loc = atomicAdd(&bodies, 1);
     stDevice(&Q.partOf[id], min(loc, 0xFFFFF));
     if (loc < Q.cap) Q.partIds[loc] = id;
@@ -1029,12 +1049,10 @@ __device__ __forceinline__ void partSingle(const PartList& Q, const PD_G int2* e
   for (int k = r0 + (int)threadIdx.x; k < r1; k += blockDim.x) {
     const int2 ab = ends[k];
     const int c = classOf(cs, Q.numColors, k);
-    const int e = first[c] + k - cs.s[c];
+    const int e = table[c].x + k - cs.s[c];
     Q.ent[e] = make_int4(k, code(ab.x) | (ab.y >= 0 ? code(ab.y) : PT_NONE) << 16, ab.x, ab.y);
     Q.nxt[e] = make_int2(0, 0);
   }
-  for (int c = threadIdx.x; c < Q.numColors; c += blockDim.x)
-    Q.bkt[c] = make_int4(first[c], 0, cs.s[c + 1] - cs.s[c], 0);
   if (threadIdx.x == 0) Q.partCnt[0] = bodies;
   __syncthreads();
 }
@@ -1061,16 +1079,17 @@ __device__ __forceinline__ void vStageAlone(const Dev& D, const Params& P, const
   vSweepLoop<1>(D, P, cs, numColors, S.stabIters, S.stabThr, S.stabThr, S.stabStop, S.stabCount, sh);
 }
 template <int MODE, bool GLOB>
-__global__ __launch_bounds__(PT_THREADS) void k_vsolve_lds(const Dev* __restrict__ Dp, Params P,
+__global__ __launch_bounds__(PT_V_THREADS) void k_vsolve_lds(const Dev* __restrict__ Dp, Params P,
                                                              ClassStarts cs, VStage S, PartList Q,
                                                              PartSync Y) {
   const Dev& D = *Dp;
   extern __shared__ double2 ptBody[];
-  __shared__ PartChunks ch;
-  __shared__ unsigned long long sh[PT_WAVES];
+  __shared__ unsigned long long sh[PT_V_THREADS / 64];
   __shared__ int go;
   const int me = blockIdx.x, parts = Q.numParts, tid = threadIdx.x;
-  if (parts == 1) partSingle(Q, D.vAB, cs, ch.base);
+  double* const body = reinterpret_cast<double*>(ptBody);
+  int4* const table = reinterpret_cast<int4*>(ptBody + (Q.cap * 6 + 1) / 2);
+  if (parts == 1) partSingle(Q, D.vAB, cs, table);
   const bool fits = GLOB || Q.partCnt[me] <= Q.cap;
   if (!partCheckIn(Y, me, parts, fits, &go)) {
     if (tid == 0 && !fits) stDevice(Y.over, 1);
@@ -1079,13 +1098,12 @@ __global__ __launch_bounds__(PT_THREADS) void k_vsolve_lds(const Dev* __restrict
     vStageAlone<MODE>(D, P, cs, Q.numColors, S, sh);
     return;
   }
-  double* const body = reinterpret_cast<double*>(ptBody);
   const int nb = min(Q.partCnt[me], Q.cap);
   const VelPart rows(D, P, Q);
   for (int s = tid; s < nb; s += blockDim.x)
     rows.globalLoad(Q.partIds[me * Q.cap + s], body + 6 * s);
-  chunksLoad(Q, me, ch);
-  PartRun<VelPart, GLOB> run(rows, Q, Y, ch, body);
+  tableLoad<PT_V_THREADS / 64>(Q, me, table);
+  PartRun<VelPart, GLOB> run(rows, Q, Y, table, body);
   run.sendRows(run.pass + 1, false);
   unsigned red = Y.seq0;
   if (S.warm) (void)run.template sweep<0>(0.0);
@@ -1118,11 +1136,12 @@ __global__ __launch_bounds__(PT_THREADS) void k_vsolve_lds(const Dev* __restrict
     ++run.pass;
     __syncthreads();
     run.sendRows(run.pass, true);
-    for (int c = 0; c < Q.numColors; ++c)
-      for (int j = chunkFirst(ch, c, run.wave); j * PT_CHUNK < ch.count[c]; j += PT_WAVES) {
+    for (int c = 0; c < Q.numColors; ++c) {
+      const int4 t = table[c];
+      for (int j = run.firstChunk(t.w); j * PT_CHUNK < t.z; j += PT_V_THREADS / 64) {
         const int at = j * PT_CHUNK + run.sub;
-        const bool live = at < ch.count[c];
-        const int4 en = Q.ent[ch.first[c] + min(at, ch.count[c] - 1)];
+        const bool live = at < t.z;
+        const int4 en = Q.ent[t.x + min(at, t.z - 1)];
         double x[6] = {0, 0, 0, 0, 0, 0};
         run.state(live, en.x, en.y, run.isB ? en.w : en.z, x);
         const d3 v{x[0], x[1], x[2]};
@@ -1133,6 +1152,7 @@ __global__ __launch_bounds__(PT_THREADS) void k_vsolve_lds(const Dev* __restrict
         *fl = sideFlags(D, make_int2(en.z, en.w), *fl, D.vVn0[en.x], v, vo, S.gHat, S.riseThr,
                         S.approachThr);
       }
+    }
     __syncthreads();  // (both lanes of a row read the flags next)
     run.start();  // (the rows have new flags)
     run.sendRows(run.pass + 1, false);
@@ -1145,7 +1165,7 @@ __global__ __launch_bounds__(PT_THREADS) void k_vsolve_lds(const Dev* __restrict
 // Position rows (posRow with the two bodies in two lanes, the odd one's normal negated): the state
 // is the predicted position.
 struct PosPart {
-  static constexpr int ND = 3;
+  static constexpr int ND = 3, THREADS = PT_P_THREADS;
   struct Row {
     d3 n, r;
     double wTotal, m, lam, lam0;  // (lam0: as loaded, see VelPart)
@@ -1202,19 +1222,22 @@ struct PosPart {
     if (!isB && (dirty & DIRTY_LAM) && (l & 0xFFFF) != PT_REMOTE) pLam[k] = w.lam;
   }
 };
-// the position loop (strict stop: residual < tol)
+// the position loop (strict stop: residual < tol); `gate` (optional): a flag that makes it return at
+// once
 template <bool GLOB>
-__global__ __launch_bounds__(PT_THREADS) void k_psolve_lds(const Dev* __restrict__ Dp,
+__global__ __launch_bounds__(PT_P_THREADS) void k_psolve_lds(const Dev* __restrict__ Dp,
                                                              ClassStarts cs, int iters, double tol,
                                                              int* stop, int* count, PartList Q,
-                                                             PartSync Y) {
+                                                             PartSync Y, const int* gate) {
   const Dev& D = *Dp;
   extern __shared__ double2 ptBody[];
-  __shared__ PartChunks ch;
-  __shared__ unsigned long long sh[PT_WAVES];
+  if (gate && *gate) return;
+  __shared__ unsigned long long sh[PT_P_THREADS / 64];
   __shared__ int go;
   const int me = blockIdx.x, parts = Q.numParts, tid = threadIdx.x;
-  if (parts == 1) partSingle(Q, D.pAB, cs, ch.base);
+  double* const body = reinterpret_cast<double*>(ptBody);
+  int4* const table = reinterpret_cast<int4*>(ptBody + (Q.cap * 3 + 1) / 2);
+  if (parts == 1) partSingle(Q, D.pAB, cs, table);
   const bool fits = GLOB || Q.partCnt[me] <= Q.cap;
   if (!partCheckIn(Y, me, parts, fits, &go)) {
     if (tid == 0 && !fits) stDevice(Y.over, 1);
@@ -1223,13 +1246,12 @@ __global__ __launch_bounds__(PT_THREADS) void k_psolve_lds(const Dev* __restrict
     pSweepLoop(D, cs, Q.numColors, iters, tol, stop, count, sh);
     return;
   }
-  double* const body = reinterpret_cast<double*>(ptBody);
   const int nb = min(Q.partCnt[me], Q.cap);
   const PosPart rows(D);
   for (int s = tid; s < nb; s += blockDim.x)
     rows.globalLoad(Q.partIds[me * Q.cap + s], body + 3 * s);
-  chunksLoad(Q, me, ch);
-  PartRun<PosPart, GLOB> run(rows, Q, Y, ch, body);
+  tableLoad<PT_P_THREADS / 64>(Q, me, table);
+  PartRun<PosPart, GLOB> run(rows, Q, Y, table, body);
   run.sendRows(run.pass + 1, false);
   unsigned long long M = 0;
   int n = 0;
@@ -1248,6 +1270,120 @@ __global__ __launch_bounds__(PT_THREADS) void k_psolve_lds(const Dev* __restrict
   __syncthreads();
   for (int s = tid; s < nb; s += blockDim.x)
     rows.globalStore(Q.partIds[me * Q.cap + s], body + 3 * s);
+}
+
+// ---- contact class 62 as a chain ------------------------------------------------------------
+// The rows of one body follow one another in row order in this class, so it is a chain of waves of
+// body-disjoint rows, for shell shapes (the many contacts of one pair) hundreds of them with a few
+// dozen rows each.  With every slot's position in LDS one wavefront walks the chain, a row per lane:
+// its LDS accesses are ordered without a barrier.  The rows of the next CHAIN_AHEAD steps are in
+// registers or in flight and the entries of as many after them: a step's dependent arithmetic is
+// ~450 clocks, a load ~1300.
+constexpr int CHAIN_AHEAD = 4;
+constexpr int CHAIN_THREADS = 256;  // (all of them move the positions)
+constexpr int CHAIN_SLOTS = 6400;
+inline int chainLdsBytes(int slots, int steps) { return slots * 24 + steps * 8; }
+// entries in wave order: (row, slot A, slot B or -1, 0)
+__global__ __launch_bounds__(TPB) void k_chain_entries(const Dev* __restrict__ Dp, const int* perm,
+                                                       int count, int4* ent) {
+  const Dev& D = *Dp;
+  const int i = gtid();
+  if (i >= count) return;
+  const int k = perm[i];
+  const int2 ab = D.pAB[k];
+  ent[i] = make_int4(k, ab.x, ab.y, 0);
+}
+struct ChainRow {
+  double4 n, rA, rB;
+  double lam;
+  int k, a, b;
+};
+__device__ __forceinline__ void chainLoad(const Dev& D, int4 e, ChainRow& w) {
+  w.k = e.x;
+  w.a = e.y;
+  w.b = e.z;
+  w.n = D.pN[e.x];
+  w.rA = D.pRA[e.x];
+  w.rB = D.pRB[e.x];
+  w.lam = D.pLam[e.x];
+}
+// posRow on positions in LDS
+__device__ __forceinline__ double chainRow(const Dev& D, const ChainRow& w, double* body) {
+  const bool hasB = w.b >= 0;
+  double* const a = body + 3 * w.a;
+  double* const b = body + 3 * (hasB ? w.b : w.a);
+  const d3 pA{a[0], a[1], a[2]}, pB{b[0], b[1], b[2]};
+  const d3 n = xyz(w.n);
+  d3 q = add3(pB, xyz(w.rB));
+  if (!hasB) q = xyz(w.rB);
+  const double C = dot3(sub3(add3(pA, xyz(w.rA)), q), n);
+  if (C >= 0.0) return 0.0;
+  if (w.n.w < 1e-6) return 0.0;
+  const double dLambda = -C / w.n.w;
+  D.pLam[w.k] = w.lam + dLambda;
+  a[0] = pA.x + n.x * dLambda * w.rA.w;
+  a[1] = pA.y + n.y * dLambda * w.rA.w;
+  a[2] = pA.z + n.z * dLambda * w.rA.w;
+  if (hasB) {
+    b[0] = pB.x + -n.x * dLambda * w.rB.w;
+    b[1] = pB.y + -n.y * dLambda * w.rB.w;
+    b[2] = pB.z + -n.z * dLambda * w.rB.w;
+  }
+  return -C;
+}
+// steps: (first entry, rows), at most 64 rows of one wave each
+__global__ __launch_bounds__(CHAIN_THREADS) void k_psweep_chain(const Dev* __restrict__ Dp,
+                                                                const int4* ent, const int2* steps,
+                                                                int numSteps, int numSlots,
+                                                                const int* stop) {
+  const Dev& D = *Dp;
+  extern __shared__ double2 ptBody[];
+  if (*stop) return;
+  double* const body = reinterpret_cast<double*>(ptBody);
+  int2* const st = reinterpret_cast<int2*>(body + 3 * numSlots);
+  for (int i = threadIdx.x; i < numSlots; i += CHAIN_THREADS) {
+    const double4 p = D.posPred[i];
+    body[3 * i] = p.x;
+    body[3 * i + 1] = p.y;
+    body[3 * i + 2] = p.z;
+  }
+  for (int i = threadIdx.x; i < numSteps; i += CHAIN_THREADS) st[i] = steps[i];
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    const int lane = (int)threadIdx.x;
+    auto entry = [&](int s) {
+      const int2 t = st[min(s, numSteps - 1)];
+      return ent[t.x + min(lane, t.y - 1)];
+    };
+    ChainRow w[CHAIN_AHEAD];
+    int4 e[CHAIN_AHEAD];
+    unsigned long long m = 0;
+#pragma unroll
+    for (int q = 0; q < CHAIN_AHEAD; ++q) chainLoad(D, entry(q), w[q]);
+#pragma unroll
+    for (int q = 0; q < CHAIN_AHEAD; ++q) e[q] = entry(CHAIN_AHEAD + q);
+    for (int s = 0; s < numSteps; s += CHAIN_AHEAD) {
+#pragma unroll
+      for (int q = 0; q < CHAIN_AHEAD; ++q) {
+        if (s + q < numSteps && lane < st[s + q].y) {
+          const unsigned long long a = dbits(chainRow(D, w[q], body));
+          m = a > m ? a : m;
+        }
+        __builtin_amdgcn_wave_barrier();
+        chainLoad(D, e[q], w[q]);
+        e[q] = entry(s + q + 2 * CHAIN_AHEAD);
+      }
+    }
+    m = waveMaxU64(m);
+    if (lane == 0 && m) atomicMax((unsigned long long*)D.maxOverlapBits, m);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < numSlots; i += CHAIN_THREADS) {
+    PD_G double4* const p = D.posPred + i;
+    p->x = body[3 * i];
+    p->y = body[3 * i + 1];
+    p->z = body[3 * i + 2];
+  }
 }
 
 }  // namespace pd

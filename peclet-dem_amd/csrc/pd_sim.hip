@@ -201,6 +201,7 @@ struct pd_sim {
   // most workgroups
   long partRows = 256;
   int partMax = 224;
+  long partBodies = 96;     // bodies per workgroup, at least
   long partsBusy = 0;       // substeps to go before the partitioned loops are tried again ...
   long partsBusyNext = 64;  // ... after one found the device busy
   // extra slots reserved by setPositions for periodic ghosts (more are added when needed)
@@ -389,9 +390,10 @@ struct pd_sim {
                           reinterpret_cast<const void*>(&k_vsolve_lds<2, false>),
                           reinterpret_cast<const void*>(&k_vsolve_lds<2, true>),
                           reinterpret_cast<const void*>(&k_psolve_lds<false>),
-                          reinterpret_cast<const void*>(&k_psolve_lds<true>)})
+                          reinterpret_cast<const void*>(&k_psolve_lds<true>),
+                          reinterpret_cast<const void*>(&k_psweep_chain)})
       HIPCHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   std::max(PT_VBODIES * 48, PT_PBODIES * 24)));
+                                   PT_LDS_BYTES));
     ensureSlots(cap > 0 ? cap : 1, 0);
     // src/sim.hpp:318-321: the multilevel gate mask comes from the environment, default slip
     if (const char* e = std::getenv("PECLET_DEM_ML_GATES")) mlGates = std::atoi(e);
@@ -464,7 +466,7 @@ struct pd_sim {
     hXi.release(); hF.release(); hTA.release(); hTB.release(); hPrevXi.release();
     hRefPos.release(); hXiWall.release(); hWF.release(); hWT.release(); hPrevKeys.release();
     hTab.release();
-    jobV.release(); jobP.release(); partsV.release(); partsP.release(); redPart.release();
+    jobV.release(); jobP.release(); partsV.release(); partsP.release(); chainSteps.release(); chainEnt.release(); redPart.release();
     ctl.release(); supList.release(); supCnt.release(); hLevel.release(); lvlKey.release(); lvlCnt.release();
     lvlStart.release(); lvlPerm.release(); lvlChanged.release(); lvlBuckets.release();
   }
@@ -1900,6 +1902,12 @@ struct pd_sim {
     }
   };
   PartJob partsV, partsP;
+  // from this many rows on the contact class 62 is run as a chain rather than by one thread
+  static constexpr int CHAIN_MIN = 64;
+  // the contact class 62 as a chain (k_psweep_chain): steps (first entry, rows) and entries
+  DBuf<int2> chainSteps;
+  DBuf<int4> chainEnt;
+  std::vector<int2> chainStepsHost;
   static constexpr long PT_SINGLE = 4;
   static constexpr size_t PT_LINE_BYTES_MAX = 0xFFFFFF00u;  // (32-bit line offsets)
   // The partitioned loop takes rows whose classes leave out the last one (62, whose rows may share
@@ -1921,13 +1929,14 @@ struct pd_sim {
   template <bool VEL>
   void buildParts(PartJob& J, const int2* ends, const double4* posOf, int ids, int rows,
                   const ClassStarts& cs, int numColors, int cap) {
+    // (a part of fewer than ~100 bodies is all boundary: packed rings, 35 contacts a body)
     // Up to partRows x PT_SINGLE rows one workgroup holds a colour's rows at once and no states
     // travel (300 spheres, 570 + 1,010 rows: 0.49 ms per substep in one workgroup, 0.66 in
     // several); beyond, a chunk of each colour per workgroup is best (9,001 spheres at 160 / 256 /
     // 384 / 640 rows per workgroup: 1.12 / 1.09 / 1.15 / 1.30 ms).
     const int parts = rows <= PT_SINGLE * partRows
                           ? 1
-                          : (int)std::min<long>(std::min(partMax, PT_MAX_PARTS),
+                          : (int)std::min<long>(std::min<long>(partMax, 1 + ids / partBodies),
                                                 (rows + partRows - 1) / partRows);
     const int levels = partLevels(parts), cells = parts > 1 ? 1 << levels : 0;
     const long most = std::min<long>(ids, 2L * rows);
@@ -2393,7 +2402,7 @@ struct pd_sim {
       kernBegin();
       auto* const kernel = usePGS ? (partsV.global ? &k_vsolve_lds<1, true> : &k_vsolve_lds<1, false>)
                                   : (partsV.global ? &k_vsolve_lds<2, true> : &k_vsolve_lds<2, false>);
-      kernel<<<Q.numParts, PT_THREADS, Q.cap * 48, st>>>(dD, P, cs, S, Q, Y);
+      kernel<<<Q.numParts, PT_V_THREADS, partLdsBytes(Q.cap, Q.numColors, 6), st>>>(dD, P, cs, S, Q, Y);
       vBlockRec[0] = kernEnd(K_VBLOCK, nRowsV);
       vFusedRec = true;
       HIPCHECK(hipGetLastError());
@@ -2575,7 +2584,10 @@ struct pd_sim {
     const bool posParts = useGS && posLeftover == 0 && posIters > 0 && nRowsP > 0 &&
                           (posSweepsPrev > 2 || nRowsP > blockRows) &&
                           partsTake(nRowsP, numPosColors, 3, 1L << 30);
-    const bool posBatches = useGS && posLeftover == 0 && nRowsP > blockRows && !posParts;
+    const int rows62 = numPosColors == 63 ? ps[63] - ps[62] : 0;
+    const bool chainFits = rows62 >= CHAIN_MIN && partRows > 0 && blockRows > 0 &&
+                           numParticles <= CHAIN_SLOTS;
+    const bool posBatches = useGS && posLeftover == 0 && (nRowsP > blockRows || chainFits) && !posParts;
     if (nRowsP > 0)
       k_prows<<<nblk(nc), TPB, 0, st>>>(dD, nc, posBatches ? bits.p : nullptr);
     mark(ST_PSWEEP);
@@ -2598,11 +2610,11 @@ struct pd_sim {
       const PartList& Q = partsP.Q;
       kernBegin();
       auto* const kernel = partsP.global ? &k_psolve_lds<true> : &k_psolve_lds<false>;
-      kernel<<<Q.numParts, PT_THREADS, Q.cap * 24, st>>>(
-          dD, pcs, posIters, posTol, ctl.p + CTL_STOP_P, ctl.p + CTL_SWEEPS_P, Q, Y);
+      kernel<<<Q.numParts, PT_P_THREADS, partLdsBytes(Q.cap, Q.numColors, 3), st>>>(
+          dD, pcs, posIters, posTol, ctl.p + CTL_STOP_P, ctl.p + CTL_SWEEPS_P, Q, Y, nullptr);
       pBlockRec = kernEnd(K_PBLOCK, nRowsP);
       HIPCHECK(hipGetLastError());
-    } else if (posLeftover == 0 && nRowsP <= blockRows) {
+    } else if (posLeftover == 0 && !posBatches) {
       if (posIters > 0) {
         kernBegin();
         k_psolve_block<<<1, BLOCK_SOLVER_THREADS, 0, st>>>(dD, classStarts(ps), numPosColors,
@@ -2620,14 +2632,29 @@ struct pd_sim {
       int cFrom = numPosColors;
       while (cFrom > 0 && ps[numPosColors] - ps[cFrom - 1] <= posTailRows) --cFrom;
       const ClassStarts pcs = classStarts(ps);
-      int waves62 = 0;
-      if (numPosColors == 63 && ps[63] - ps[62] >= std::max(1L, waveMinRows)) {
+      int waves62 = 0, chain = 0;
+      if (rows62 > 0 && (chainFits || rows62 >= waveMinRows)) {
         cFrom = 63;  // colour 62 leaves the tail launch: it runs in waves
-        const int cnt62 = ps[63] - ps[62];
+        const int cnt62 = rows62;
         std::vector<int2> ends(cnt62);
         readN(ends.data(), pAB.p + ps[62], cnt62);
         waves62 = serialClassWaves(ends.data(), cnt62, numParticles, ps[62], pWavePerm,
                                    pWaveStart);
+        // with every slot in one workgroup's LDS: one wavefront walks the waves as a chain (3,001
+        // packed rings, 911 waves of 42,081 rows: 1.27 ms per sweep in the launch and segments
+        // below, 0.44 ms in the chain)
+        chainStepsHost.clear();
+        for (int w = 0; w < waves62; ++w)
+          for (int b = waveCnt[w]; b < waveCnt[w + 1]; b += 64)
+            chainStepsHost.push_back(make_int2(b, std::min(64, waveCnt[w + 1] - b)));
+        if (chainFits && chainLdsBytes(
+                numParticles, (int)chainStepsHost.size()) <= PT_LDS_BYTES) {
+          chain = (int)chainStepsHost.size();
+          chainSteps.ensure(chain, st);
+          chainEnt.ensure(cnt62, st);
+          writeN(chainSteps.p, chainStepsHost.data(), chain);
+          k_chain_entries<<<nblk(cnt62), TPB, 0, st>>>(dD, pWavePerm.p, cnt62, chainEnt.p);
+        }
         pWaveStartHost.assign(waveCnt.begin(), waveCnt.begin() + waves62 + 1);
         pWaveSegs.clear();
         for (int w = 0; w < waves62; ++w) {
@@ -2638,15 +2665,30 @@ struct pd_sim {
             pWaveSegs.push_back(make_int3(w, w + 1, big ? 1 : 0));
         }
       }
+      // beside a chain, the other classes of a sweep run in one launch over a partition (3,001
+      // packed rings, 62 classes: 257 us per sweep in a launch each, 170 us in one)
+      const bool partSweeps = chain > 0 && partsTake(ps[62], 62, 3, 1L << 30);
+      if (partSweeps)
+        buildParts<false>(partsP, pAB.p, posPred.p, numParticles, ps[62], pcs, 62, PT_PBODIES);
       int done = 0, batch = std::max(1, std::min(posIters, posSweepsPrev));
       // (the residual was cleared by the rows launch)
       while (done < posIters) {
         const int b = std::min(batch, posIters - done);
         for (int j = 0; j < b; ++j) {
-          for (int c = 0; c < cFrom; ++c) {
+          if (partSweeps) {
+            const PartSync Y = partSync(partsP, ps[62], 3, 2, false);
+            const PartList& Q = partsP.Q;
+            auto* const kernel = partsP.global ? &k_psolve_lds<true> : &k_psolve_lds<false>;
+            kernel<<<Q.numParts, PT_P_THREADS, partLdsBytes(Q.cap, Q.numColors, 3), st>>>(
+                dD, pcs, 1, -1.0, ctl.p + CTL_DUMP, ctl.p + CTL_DUMP, Q, Y, ctl.p + CTL_STOP_P);
+          }
+          for (int c = partSweeps ? 62 : 0; c < cFrom; ++c) {
             const int cb = ps[c], ce = ps[c + 1];
             if (ce <= cb) continue;
-            if (c == 62 && waves62 > 0) {
+            if (c == 62 && chain > 0) {
+              k_psweep_chain<<<1, CHAIN_THREADS, chainLdsBytes(numParticles, chain), st>>>(
+                  dD, chainEnt.p, chainSteps.p, chain, numParticles, ctl.p + CTL_STOP_P);
+            } else if (c == 62 && waves62 > 0) {
               for (const int3 g : pWaveSegs) {
                 if (g.z) {
                   const int wb = pWaveStartHost[g.x], we = pWaveStartHost[g.y];
@@ -4059,6 +4101,9 @@ int pd_set_tuning(pd_sim* s, const char* name, long value) {
     } else if (k == "partition_rows") {
       if (value < 0) throw ArgError("partition_rows must be >= 0");
       s->partRows = value;
+    } else if (k == "partition_bodies") {
+      if (value < 1) throw ArgError("partition_bodies must be >= 1");
+      s->partBodies = value;
     } else if (k == "partition_workgroups") {
       if (value < 1 || value > PT_MAX_PARTS)
         throw ArgError("partition_workgroups must be in [1, " + std::to_string(PT_MAX_PARTS) + "]");

@@ -71,3 +71,31 @@ def test_partition_equals_the_launches_per_colour(hip_lib, kind, n, tunings):
     for other in runs[1:]:
         for a, b in zip(runs[0], other):
             assert np.array_equal(a, b) if isinstance(a, np.ndarray) else a == b
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tuning", [{}, {"partition_bodies": 20}, {"partition_rows": 0}],
+                         ids=["chain", "more-parts", "launches"])
+def test_last_contact_class_as_a_chain(hip_lib, tuning):
+    # packed hollow cylinders with a dense shell: hundreds of rows in the contact class whose rows
+    # share bodies, walked by one wavefront beside the other classes' partition, or in launches
+    from oracle_binding import oracle_sim
+    from peclet.dem import Simulation
+    from peclet.dem.workloads import cylinder_pack, setup_cylinder_bed
+
+    n = 300
+    bed = cylinder_pack(n, 0.0274, 3)
+    h = setup_cylinder_bed(Simulation(n), bed, 5e-6, 0.4, 0.2)
+    for key, value in tuning.items():
+        h.set_tuning(key, value)
+    r = setup_cylinder_bed(oracle_sim(n), bed, 5e-6, 0.4, 0.2)
+    for k in range(2):
+        print(n, tuning, k, flush=True)
+        h.step(5e-6)
+        r.step(5e-6)
+        for name in ("get_positions", "get_velocities", "get_angular_velocities"):
+            assert np.array_equal(getattr(h, name)(), getattr(r, name)()), (k, name)
+        assert h.get_stats()["sweeps_pos"] == r.get_stats()["sweeps_pos"]
+        colours = h.debug_contact_colors()
+        assert np.array_equal(colours, r.debug_contact_colors())
+    assert (colours == 62).sum() > 64
