@@ -99,3 +99,11 @@ def test_last_contact_class_as_a_chain(hip_lib, tuning):
         colours = h.debug_contact_colors()
         assert np.array_equal(colours, r.debug_contact_colors())
     assert (colours == 62).sum() > 64
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("skin", [100, 1])
+def test_candidate_list_left_out_after_failures(hip_lib, skin):
+    # images that come and go, and a skin that every step outruns: lists that fail at their first
+    # reuse, the substeps that go without one, and the next list
+    run_pair("bed_periodic", 300, 50, tuning={"candidate_skin_permille": skin})
