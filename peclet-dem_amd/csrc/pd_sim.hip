@@ -181,8 +181,10 @@ struct pd_sim {
   double hertzFrac = 0.5;
   int hNumPairs = -1, hPrevCount = 0, hNumWallCand = 0;
   DBuf<int2> hPairs;
-  DBuf<int> hIStart, hJStart, hJList, hJCnt, hWStart, hWCand, hWCnt;
-  DBuf<double4> hXi, hF, hTA, hTB, hPrevXi, hRefPos, hXiWall, hWF, hWT;
+  DBuf<int> hIStart, hJStart, hJList, hJPos, hJCnt, hWStart, hWCand, hWCnt;
+  DBuf<double2> hRecI, hRecJ;
+  DBuf<unsigned char> hActI, hActJ;
+  DBuf<double4> hXi, hPrevXi, hRefPos, hXiWall, hWF, hWT;
   DBuf<unsigned long long> hPrevKeys;
   DBuf<HzTab> hTab;
   HzDev Z{};
@@ -462,8 +464,9 @@ struct pd_sim {
     frCnt.release();
     jC.release(); jF.release(); jIncCnt.release(); jIncStart.release(); jIncList.release();
     wallGridD.release(); sdfGridD.release(); hPairs.release(); hIStart.release(); hJStart.release();
-    hJList.release(); hJCnt.release(); hWStart.release(); hWCand.release(); hWCnt.release();
-    hXi.release(); hF.release(); hTA.release(); hTB.release(); hPrevXi.release();
+    hJList.release(); hJPos.release(); hJCnt.release(); hWStart.release(); hWCand.release(); hWCnt.release();
+    hXi.release(); hRecI.release(); hRecJ.release(); hActI.release(); hActJ.release();
+    hPrevXi.release();
     hRefPos.release(); hXiWall.release(); hWF.release(); hWT.release(); hPrevKeys.release();
     hTab.release();
     jobV.release(); jobP.release(); partsV.release(); partsP.release(); chainSteps.release(); chainEnt.release(); redPart.release();
@@ -2837,7 +2840,8 @@ struct pd_sim {
   // ---------------------------------------------------------------- Hertz–Mindlin engine
   void refreshHz() {
     Z.pairs = hPairs.p; Z.iStart = hIStart.p; Z.jStart = hJStart.p; Z.jList = hJList.p;
-    Z.xi = hXi.p; Z.f = hF.p; Z.tA = hTA.p; Z.tB = hTB.p; Z.prevKeys = hPrevKeys.p;
+    Z.jPos = hJPos.p; Z.xi = hXi.p; Z.actI = hActI.p; Z.actJ = hActJ.p;
+    Z.recI = hRecI.p; Z.recJ = hRecJ.p; Z.prevKeys = hPrevKeys.p;
     Z.prevXi = hPrevXi.p; Z.refPos = hRefPos.p; Z.wStart = hWStart.p; Z.wCand = hWCand.p;
     Z.xiWall = hXiWall.p; Z.wf = hWF.p; Z.wt = hWT.p; Z.wallGrid = wallGridD.p; Z.tab = hTab.p;
   }
@@ -2910,10 +2914,12 @@ struct pd_sim {
     broadphase(P);
     hPairs.ensure(np + 1, st);
     hXi.ensure(np + 1, st);
-    hF.ensure(np + 1, st);
-    hTA.ensure(np + 1, st);
-    hTB.ensure(np + 1, st);
+    hRecI.ensure(3 * (size_t)np + 1, st);
+    hRecJ.ensure(3 * (size_t)np + 1, st);
+    hActI.ensure(np + 1, st);
+    hActJ.ensure(np + 1, st);
     hJList.ensure(np + 1, st);
+    hJPos.ensure(np + 1, st);
     hIStart.ensure(n + 1, st);
     hJStart.ensure(n + 1, st);
     hJCnt.ensure(n + 1, st);
@@ -2978,7 +2984,7 @@ struct pd_sim {
       H = hzParams(dtH);
       if (H.numPairs > 0) {
         if (H.hasShapes) k_hz_shape_pairs<<<nblk(H.numPairs), TPB, 0, st>>>(dD, Z, H);
-        else k_hz_pairs<<<nblk(H.numPairs), TPB, 0, st>>>(dD, Z, H);
+        else k_hz_pairs<<<(H.numPairs + HZ_TILE - 1) / HZ_TILE, TPB, 0, st>>>(dD, Z, H);
       }
       if (H.numWalls > 0 && hNumWallCand > 0)
         k_hz_walls<<<nblk(hNumWallCand), TPB, 0, st>>>(dD, Z, H, hNumWallCand);
