@@ -1889,26 +1889,16 @@ struct pd_sim {
   // One partition of the rows of a sweep loop (pd_parts.hpp): the velocity rows over the reals, or
   // the position rows over the slots.
   struct PartJob {
-    DBuf<PartGrid> grid;
-    DBuf<unsigned long long> mask;
-    DBuf<int> hist, cellStart, partOf, partCnt, partIds, bktCnt, listStart, list;
-    DBuf<int4> bkt, ent;
-    DBuf<int2> rank, nxt;
-    DBuf<double> lam2;
-    DBuf<double4> lamT2;
-    DBuf<unsigned char> flag2;
-    DBuf<pu4> lines, red;
-    DBuf<unsigned> arrive;  // [PT_MAX_PARTS] check-ins, then the decision
+    DBuf<unsigned char> mem;  // the lists of Q, built anew for every loop (one allocation: a batch
+                              // of 32 small systems otherwise makes 450 more in its first step)
+    DBuf<pu4> lines;
+    DBuf<pu4> sync;           // maxima [2 x PT_MAX_PARTS], then the check-ins and the decision
     unsigned seq = 0, epoch = 0;
     bool global = false;    // a part may have more bodies than LDS slots
     bool everOver = false;  // one had, unexpectedly
     PartList Q{};
     void release() {
-      mask.release(); listStart.release(); list.release(); nxt.release();
-      grid.release(); hist.release(); cellStart.release(); partOf.release();
-      partCnt.release(); partIds.release(); bktCnt.release(); bkt.release(); ent.release();
-      rank.release(); lam2.release(); lamT2.release(); flag2.release(); lines.release();
-      red.release(); arrive.release();
+      mem.release(); lines.release(); sync.release();
     }
   };
   PartJob partsV, partsP;
@@ -1955,42 +1945,54 @@ struct pd_sim {
     const int capL = (int)std::min<long>(cap, room);
     J.global = room > cap || J.everOver;
     const int bkts = parts * std::max(1, numColors);
-    J.partOf.ensure(ids + 1, st);
-    J.partCnt.ensure(PT_MAX_PARTS + 1, st);  // (and the lists' counter)
-    J.partIds.ensure((size_t)parts * capL, st);
-    J.bktCnt.ensure(2 * bkts, st);
-    J.bkt.ensure(bkts, st);
     const long entries = (parts > 1 ? 2L : 1L) * rows + (long)PT_CHUNK * bkts;
-    J.ent.ensure(entries, st);
-    J.nxt.ensure(entries, st);
-    if (parts > 1) {
-      J.grid.ensure(1, st);
-      J.mask.ensure(ids + 1, st);
-      J.listStart.ensure(ids + 1, st);
-      J.list.ensure(2L * rows + 1, st);
-      J.hist.ensure(PT_MAX_CELLS + 1, st);
-      J.cellStart.ensure(PT_MAX_CELLS + 1, st);
-      J.rank.ensure(rows + 1, st);
-    }
-    J.red.ensure(2 * PT_MAX_PARTS, st);
-    J.arrive.ensure(PT_MAX_PARTS + 1, st);
-    if (VEL && parts > 1) {
-      J.lam2.ensure(rows, st);
-      J.lamT2.ensure(rows, st);
-      J.flag2.ensure(rows, st);
-    }
-    if (parts > 1) J.lines.ensure((size_t)rows * 4 * (VEL ? 6 : 3), st);
     PartList& Q = J.Q;
-    Q = PartList{parts, numColors, capL, J.grid.p, J.mask.p, J.listStart.p, J.list.p,
-                 J.partCnt.p + PT_MAX_PARTS, J.hist.p, J.cellStart.p, J.partOf.p, J.partCnt.p,
-                 J.partIds.p, J.bktCnt.p, J.bkt.p, J.rank.p, J.ent.p, J.nxt.p, J.lam2.p,
-                 J.lamT2.p, J.flag2.p};
+    Q = PartList{};
+    Q.numParts = parts;
+    Q.numColors = numColors;
+    Q.cap = capL;
+    // places of the lists in the allocation: called once for its size, then for the pointers
+    auto lay = [&](unsigned char* base) {
+      size_t off = 0;
+      auto take = [&](auto*& q, size_t n) {
+        using T = std::remove_reference_t<decltype(*q)>;
+        q = base ? reinterpret_cast<T*>(base + off) : nullptr;
+        off += (n * sizeof(T) + 255) & ~(size_t)255;
+      };
+      take(Q.partOf, ids + 1);
+      take(Q.partCnt, PT_MAX_PARTS + 1);  // (and the lists' counter)
+      take(Q.partIds, (size_t)parts * capL);
+      take(Q.bktCnt, 2 * bkts);
+      take(Q.bkt, bkts);
+      take(Q.ent, entries);
+      take(Q.nxt, entries);
+      if (parts > 1) {
+        take(Q.grid, 1);
+        take(Q.mask, ids + 1);
+        take(Q.listStart, ids + 1);
+        take(Q.list, 2L * rows + 1);
+        take(Q.hist, PT_MAX_CELLS + 1);
+        take(Q.cellStart, PT_MAX_CELLS + 1);
+        take(Q.rank, rows + 1);
+      }
+      if (VEL && parts > 1) {
+        take(Q.lam2, rows);
+        take(Q.lamT2, rows);
+        take(Q.flag2, rows);
+      }
+      return off;
+    };
+    J.mem.ensure(lay(nullptr), st);
+    lay(J.mem.p);
+    Q.listCnt = Q.partCnt + PT_MAX_PARTS;
+    J.sync.ensure(2 * PT_MAX_PARTS + (PT_MAX_PARTS + 1 + 3) / 4, st);
+    if (parts > 1) J.lines.ensure((size_t)rows * 4 * (VEL ? 6 : 3), st);
     if (parts > 1) {  // (a loop of one workgroup builds its partition itself)
       k_part_begin<<<nblk(std::max(std::max(ids, cells), 2 * bkts)), TPB, 0, st>>>(
           Q, gridD.p, ids, cells, levels);
       k_part_colours<<<nblk(rows), TPB, 0, st>>>(Q, ends, cs, rows);
       k_part_hist<<<nblk(ids), TPB, 0, st>>>(Q, posOf, ids);
-      scanQuiet(J.hist.p, J.cellStart.p, cells);
+      scanQuiet(Q.hist, Q.cellStart, cells);
       k_part_assign<<<(ids + 1023) / 1024, 1024, 0, st>>>(Q, posOf, ids, cells);
       k_part_count<<<(rows + 1023) / 1024, 1024, 0, st>>>(Q, ends, cs, rows);
       k_part_ranges<<<1, 1024, 0, st>>>(Q);
@@ -2004,16 +2006,15 @@ struct pd_sim {
     if (J.seq > 0xFFFFFFFFu - (unsigned long)passes - 2 || J.epoch >= 0x7FFFFFFEu) {
       // the numbers start over: no line may hold an old one
       zero(J.lines.p, J.lines.cap);
-      zero(J.red.p, J.red.cap);
-      zero(J.arrive.p, J.arrive.cap);
+      zero(J.sync.p, J.sync.cap);
       J.seq = J.epoch = 0;
     }
     Y.lines = J.lines.p;
     Y.half = (unsigned)((size_t)rows * 2 * 16 * nd);
     Y.lineBytes = 2 * Y.half;
-    Y.red = J.red.p;
-    Y.arrive = J.arrive.p;
-    Y.decision = J.arrive.p + PT_MAX_PARTS;
+    Y.red = J.sync.p;
+    Y.arrive = reinterpret_cast<unsigned*>(J.sync.p + 2 * PT_MAX_PARTS);
+    Y.decision = Y.arrive + PT_MAX_PARTS;
     Y.seq0 = J.seq;
     J.seq += (unsigned)passes + 1;
     Y.epoch = ++J.epoch;
