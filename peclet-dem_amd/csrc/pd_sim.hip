@@ -2342,7 +2342,12 @@ struct pd_sim {
                           legacyFriction;
     const bool smallV = nRowsV <= blockRows;
     // the whole velocity stage in one launch over a partition of the bodies
-    const bool fusedV = !hostLoop && velIters > 0 && ldsLoop && partsTake(nRowsV, numColors, 6, PARTS_V_ROWS);
+    // (not beside the colouring of many more contacts than rows on the other stream: 200k packed
+    // cylinders, 8.8M contacts and 0.52M rows, 47.8 ms against 4.4 ms by launches per colour,
+    // about what one workgroup alone takes; 1M poured spheres, ~1M contacts and 0.55M rows, gain)
+    const bool fusedV = !hostLoop && velIters > 0 && ldsLoop &&
+                        (nRowsV <= blockRows || nc <= 2 * PARTS_V_ROWS) &&
+                        partsTake(nRowsV, numColors, 6, PARTS_V_ROWS);
     const size_t R = nRowsV + 1;
     vAB.ensure(R, st); vN.ensure(R, st); vTA.ensure(R, st); vTB.ensure(R, st); vRA.ensure(R, st);
     vRB.ensure(R, st); vVt0.ensure(R, st); vLamT.ensure(R, st); vVn0.ensure(R, st);
@@ -2605,8 +2610,7 @@ struct pd_sim {
     // with the batched position loop ahead, the rows launch also clears its residual
     // (a loop that stops after a sweep or two does not repay building a partition)
     const bool posParts = useGS && posLeftover == 0 && posIters > 0 && nRowsP > 0 &&
-                          (posSweepsPrev > 2 || nRowsP > blockRows) &&
-                          partsTake(nRowsP, numPosColors, 3, 1L << 30);
+                          posSweepsPrev > 2 && partsTake(nRowsP, numPosColors, 3, 1L << 30);
     const int rows62 = numPosColors == 63 ? ps[63] - ps[62] : 0;
     const bool chainFits = rows62 >= CHAIN_MIN && partRows > 0 && blockRows > 0 &&
                            numParticles <= CHAIN_SLOTS;
