@@ -137,6 +137,10 @@ int pd_get_manifold_colors(pd_sim* s, int* out, int cap);
 int pd_get_ledger(pd_sim* s, uint64_t* keys, double* lambda, double* lambdaT, double* posImp,
                   int cap);                                          /* warm-start store */
 int pd_get_grounded(pd_sim* s, int* out, int n);
+/* how often each of the internal forms of a substep's parts was taken since the handle was made
+ * (no reference counterpart): candidate pair list rebuilt, reused, left out for the substep;
+ * returns the number of counters and writes at most cap of them */
+int pd_get_path_counts(pd_sim* s, long* out, int cap);
 
 /* --- host-side export ------------------------------------------------------------------- */
 int pd_export_lammps(pd_sim* s, const char* filename, int step); /* exportLammps, :1463 */

@@ -972,7 +972,7 @@ struct pd_sim {
     numReal = n;
     numParticles = n;
     hNumPairs = -1;  // particle indices changed: the Hertz pair cache is stale, :1294-1295
-    candValid = false;
+    candForget();
     hPrevCount = 0;
     std::vector<double4> P((size_t)n);
     std::vector<BodyC> B((size_t)n);
@@ -1075,14 +1075,22 @@ struct pd_sim {
   int candSlots = 0, candNumReal = -1;
   double candSkin = 0.0, candMargin = 0.0;
   double candSkinFrac = 0.1;  // skin = this x the largest radius (0: rebuild every substep)
+  // substeps that rebuilt the list, used it, went without one
   long candRebuilds = 0, candReuses = 0;
   // the list was used again since its rebuild; rebuilds running whose list was not; substeps to go
   // without one (a failed list costs its rebuild's filter and the failed check: 1M resting bed
   // 1.53 ms of broadphase per substep with a list rebuilt every time, 0.46 ms without)
   bool candReused = true;
   int candFails = 0;
-  long candSkip = 0;
+  long candSkip = 0, candSkipped = 0;
   static constexpr long CAND_SKIP_MAX = 64;
+  // a new skin or new positions: neither the list nor what its predecessors did says anything
+  void candForget() {
+    candValid = false;
+    candReused = true;
+    candFails = 0;
+    candSkip = 0;
+  }
   int lastGhosts = 0;
   DBuf<Grid> gridD;
   DBuf<int> ncellD;
@@ -2176,7 +2184,10 @@ struct pd_sim {
     // periodic bed some ghost image comes or goes in every substep)
     if (candSkip > 0) candValid = false;
     double skin = candSkip > 0 ? 0.0 : candSkinFrac * maxRad;
-    if (candSkip > 0) --candSkip;
+    if (candSkip > 0) {
+      --candSkip;
+      ++candSkipped;
+    }
     bool useCand = candValid && skin > 0.0 && candNumReal == numReal && candSkin == skin &&
                    candMargin == margin;
     int G = 0;
@@ -2222,6 +2233,7 @@ struct pd_sim {
           candSkip = std::min(CAND_SKIP_MAX, 8L << std::min(candFails, 16));
           skin = 0.0;
           candValid = false;
+          ++candSkipped;
         }
         continue;
       }
@@ -3169,7 +3181,7 @@ static TuneCfg tuneCurrent(const pd_sim* s) {
 static void tuneApply(pd_sim* s, const TuneCfg& c) {
   if ((long)std::lround(s->candSkinFrac * 1000.0) != c.skin) {
     s->candSkinFrac = c.skin / 1000.0;
-    s->candValid = false;
+    s->candForget();
   }
   s->blockRows = (int)c.rows;
   s->ldsLoop = c.lds != 0;
@@ -3190,6 +3202,7 @@ static double tuneTrial(pd_sim* s, double dt, int substeps) {
 }
 static TuneCfg tuneRun(pd_sim* s, double dt, int substeps, double* bestMs) {
   TuneCfg cur = tuneCurrent(s);
+  s->candForget();  // (every skin starts its trial alike)
   double best = tuneTrial(s, dt, substeps);
   const long skins[] = {0, 50, 100, 200, 400};
   const long rows[] = {0, 2048, 16384, 65536};
@@ -3959,6 +3972,12 @@ int pd_get_ledger(pd_sim* s, uint64_t* keys, double* lambda, double* lambdaT, do
   }
   return s->prevCount;
 }
+int pd_get_path_counts(pd_sim* s, long* out, int cap) {
+  const long v[] = {s->candRebuilds, s->candReuses, s->candSkipped};
+  const int n = (int)(sizeof(v) / sizeof(v[0]));
+  for (int k = 0; out && k < n && k < cap; ++k) out[k] = v[k];
+  return n;
+}
 int pd_get_grounded(pd_sim* s, int* out, int n) {
   if (out) guard([&] { s->readN(out, s->ground.p, std::min(n, s->numReal)); });
   return s->numReal;
@@ -4141,7 +4160,7 @@ int pd_set_tuning(pd_sim* s, const char* name, long value) {
     } else if (k == "candidate_skin_permille") {
       if (value < 0) throw ArgError("candidate_skin_permille must be >= 0");
       s->candSkinFrac = std::min<long>(value, 100000) / 1000.0;
-      s->candValid = false;
+      s->candForget();
     } else if (k == "slot_headroom") {
       if (value < 0) throw ArgError("slot_headroom must be >= 0");
       s->slotHeadroom = std::min<long>(value, 1L << 30);

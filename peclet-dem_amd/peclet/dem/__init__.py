@@ -615,6 +615,14 @@ class Simulation:
         self._b.get_grounded(self._h, out.ctypes.data_as(C.POINTER(C.c_int)), n)
         return out
 
+    PATHS = ("list_rebuilt", "list_reused", "list_left_out")
+
+    def debug_paths(self):
+        """How often each internal form of a substep's parts was taken (extension)."""
+        out = (C.c_long * len(self.PATHS))()
+        assert self._b.get_path_counts(self._h, out, len(out)) == len(out)
+        return dict(zip(self.PATHS, out))
+
     # ------------------------------------------------------------------ export (host side)
     def export_lammps(self, filename, step):
         self._chk(self._b.export_lammps(self._h, os.fsencode(filename), int(step)))

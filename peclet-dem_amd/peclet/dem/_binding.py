@@ -134,6 +134,7 @@ PRODUCT_SIGNATURES = {
     "get_stats_log": (_i, [_p, C.POINTER(Stats), _i]),
     "kernel_name": (C.c_char_p, [_i]),
     "set_tuning": (_i, [_p, C.c_char_p, C.c_long]),
+    "get_path_counts": (_i, [_p, C.POINTER(C.c_long), _i]),
     "export_sdf": (_i, [_p, C.c_char_p, _i, _i, _i]),
     "read_device": (_i, [_p, _p, _p, C.c_size_t]),
     "write_device": (_i, [_p, _p, _p, C.c_size_t]),

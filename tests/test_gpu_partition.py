@@ -107,3 +107,37 @@ def test_candidate_list_left_out_after_failures(hip_lib, skin):
     # images that come and go, and a skin that every step outruns: lists that fail at their first
     # reuse, the substeps that go without one, and the next list
     run_pair("bed_periodic", 300, 50, tuning={"candidate_skin_permille": skin})
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("change", ["skin", "positions", "autotune"])
+def test_candidate_list_returns_after_a_change(hip_lib, change):
+    # a skin that every step outruns, until the list is left out; a new skin, new positions or the
+    # autotuner's trials start with a list at once
+    from peclet.dem import Simulation
+    from scenes import apply_scene, make_scene
+
+    scene = make_scene("bed_periodic", 300, 3)
+    scene["vel"] = scene["vel"] + np.array([3.0, 2.0, 0.0])
+    h = apply_scene(Simulation(300), scene)
+    h.set_tuning("candidate_skin_permille", 1)
+    for _ in range(16):
+        h.step(scene["dt"])
+        if h.debug_paths()["list_left_out"] >= 2:
+            break
+    before = h.debug_paths()
+    assert before["list_left_out"] >= 2
+    if change == "autotune":
+        cfg, ms = h.autotune(scene["dt"], substeps=2, use_cache=False)
+        # every trial with a skin of its own builds one: the current, four tried, the choice
+        assert h.debug_paths()["list_rebuilt"] >= before["list_rebuilt"] + 4
+    else:
+        if change == "skin":
+            h.set_tuning("candidate_skin_permille", 400)
+        else:
+            h.set_positions(scene["pos"])
+        h.step(scene["dt"])
+        after = h.debug_paths()
+        assert after["list_rebuilt"] == before["list_rebuilt"] + 1
+        assert after["list_left_out"] == before["list_left_out"]
+    h.close()
