@@ -262,7 +262,10 @@ int pd_set_timing(pd_sim* s, int level);
  * as is block_solver_rows 0): the rows per workgroup of the partitioned velocity and position
  * loops, four times as many for a loop in one workgroup; "partition_workgroups" (default 224, at
  * most 256): the most workgroups of one, "partition_bodies" (default 96): the fewest bodies per
- * workgroup; "vsweep_waves" = 3 (default)
+ * workgroup; "partition_wait_polls" (default and maximum 2^22, at least 128): the polls after which
+ * a workgroup gives up waiting for another's body states, upon which the step fails and the handle
+ * steps again only after pd_set_positions; "partition_absent" = 2 (default 0) makes one workgroup
+ * leave them waiting, for tests of that; "vsweep_waves" = 3 (default)
  * or 4 selects the per-colour PGS sweep compiled for that many waves per SIMD (4: at most 128
  * VGPRs, with some register spilling); "velocity_pack_bodies" = 1 (default) lets the per-colour
  * velocity launches read each body's velocity and constants from one 128-byte record packed for

@@ -34,7 +34,8 @@
 // within a bounded time (other work holds the compute units) they agree, through one compare-and-
 // swap, to leave, and workgroup 0 runs the loop alone from global memory.  Once all have checked in
 // every wait ends, since a workgroup never leaves before the loop does; the waits are bounded all
-// the same and a wait that runs out raises an error on the host.
+// the same, in polls and not by a clock (a process may be suspended for any time, and its polls
+// with it), and a wait that runs out raises an error on the host.
 // Bound: a colour pass is one row's dependent arithmetic, ~430 FP64 operations at 5-8 clocks plus
 // the loads of its bodies from LDS, 1.7-2 us, and for a row between parts what the hop leaves of
 // ~1.5 us; ~200 velocity and ~110 position passes make a substep.  Substeps of resting beds, MI355X,
@@ -111,9 +112,11 @@ struct PartSync {
   int* over;         // set when a part had more bodies than LDS slots
   int* fail;         // set when a wait ran out
   int refuse;        // 1: leave at the check-in (tests)
+  int absent;        // 2: the last workgroup leaves after the check-in (tests)
+  int waitPolls;     // polls after which a wait has run out
 };
-constexpr long PT_CHECKIN_TICKS = 200000;     // 2 ms of the 100 MHz clock
-constexpr long PT_WAIT_TICKS = 200000000;     // 2 s
+constexpr long PT_CHECKIN_TICKS = 200000;  // 2 ms of the 100 MHz clock
+constexpr int PT_WAIT_POLLS = 1 << 22;     // (a poll takes 0.5-1 us)
 
 // device-scope accesses
 template <class T>
@@ -386,21 +389,18 @@ __device__ __forceinline__ void lineSend(__amdgpu_buffer_rsrc_t r, unsigned off,
 __device__ __forceinline__ double lineValue(pu4 w) {
   return bitsd((unsigned long long)w.z << 32 | w.x);
 }
-// the clock and error check of a wait, every 128 polls; true: give up
-__device__ __forceinline__ bool waitOver(int polls, long& t0, int* fail) {
+// the error check of a wait, every 128 polls; true: give up
+__device__ __forceinline__ bool waitOver(int polls, int most, int* fail) {
   if ((polls & 127) != 127) return false;
   if (ldDevice(fail)) return true;
-  const long t = (long)wall_clock64();
-  if (polls == 127) t0 = t;
-  if (t - t0 < PT_WAIT_TICKS) return false;
+  if (polls < most) return false;
   stDevice(fail, 1);
   return true;
 }
 // ND doubles sent with `seq`, by the lanes with `need`; every lane of the wave calls it
 template <int ND>
 __device__ __forceinline__ void lineRecv(__amdgpu_buffer_rsrc_t r, unsigned off, unsigned seq,
-                                         bool need, double* x, int* fail) {
-  long t0 = 0;
+                                         bool need, double* x, int most, int* fail) {
   bool wait = need;
   for (int n = 0;; ++n) {
     if (wait) {
@@ -414,7 +414,7 @@ __device__ __forceinline__ void lineRecv(__amdgpu_buffer_rsrc_t r, unsigned off,
         x[q] = lineValue(w[q]);
       }
     }
-    if (!__any(wait) || waitOver(n, t0, fail)) break;
+    if (!__any(wait) || waitOver(n, most, fail)) break;
   }
 }
 // every workgroup is running, and `fits` in all of them: true in all of them, or false in all
@@ -459,7 +459,7 @@ __device__ __forceinline__ unsigned long long partMax(unsigned long long m, cons
   if (threadIdx.x == 0) lineSend(r, me * 16, bitsd(M), seq);
   double x = 0.0;
   const bool need = (int)threadIdx.x < parts;
-  lineRecv<1>(r, threadIdx.x * 16, seq, need, &x, Y.fail);
+  lineRecv<1>(r, threadIdx.x * 16, seq, need, &x, Y.waitPolls, Y.fail);
   return blockMaxAll(need ? dbits(x) : 0ull, sh);
 }
 
@@ -536,6 +536,7 @@ struct PartRun {
   const int4* const ent;
   const int* const nxt;  // [entries][2]
   int* const fail;
+  const int waitPolls;
   const unsigned half;
   const int4* const table;  // LDS [numColors]
   double* const body;       // LDS [cap][ND]
@@ -552,7 +553,8 @@ struct PartRun {
 
   __device__ __forceinline__ PartRun(const R& r, const PartList& q, const PartSync& y,
                                      const int4* t, double* b)
-      : rows(r), numColors(q.numColors), ent(q.ent), nxt((const int*)q.nxt), fail(y.fail), half(y.half), table(t), body(b),
+      : rows(r), numColors(q.numColors), ent(q.ent), nxt((const int*)q.nxt), fail(y.fail),
+        waitPolls(y.waitPolls), half(y.half), table(t), body(b),
         lines(lineRsrc(y.lines, y.lineBytes)), pass(y.seq0) {
     wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     sub = (int)(threadIdx.x & 63) >> 1;
@@ -658,7 +660,7 @@ struct PartRun {
     const bool remote = live && loc == PT_REMOTE;
     if (live && !remote && loc != PT_NONE) bodyLoad(loc, id, x);
     if (__any(remote))
-      lineRecv<ND>(lines, remote ? lineAt(2 * k + (isB ? 1 : 0), pass) : 0u, pass, remote, x, fail);
+      lineRecv<ND>(lines, remote ? lineAt(2 * k + (isB ? 1 : 0), pass) : 0u, pass, remote, x, waitPolls, fail);
   }
   // send, for pass `seq`, the states of this wave's rows between parts: all of them, or of those
   // that are their body's first row in a pass (what the rows before do not send)
@@ -1098,6 +1100,7 @@ __global__ __launch_bounds__(PT_V_THREADS) void k_vsolve_lds(const Dev* __restri
     vStageAlone<MODE>(D, P, cs, Q.numColors, S, sh);
     return;
   }
+  if (Y.absent == 2 && me != 0 && me == parts - 1) return;
   const int nb = min(Q.partCnt[me], Q.cap);
   const VelPart rows(D, P, Q);
   for (int s = tid; s < nb; s += blockDim.x)
@@ -1246,6 +1249,7 @@ __global__ __launch_bounds__(PT_P_THREADS) void k_psolve_lds(const Dev* __restri
     pSweepLoop(D, cs, Q.numColors, iters, tol, stop, count, sh);
     return;
   }
+  if (Y.absent == 2 && me != 0 && me == parts - 1) return;
   const int nb = min(Q.partCnt[me], Q.cap);
   const PosPart rows(D);
   for (int s = tid; s < nb; s += blockDim.x)

@@ -204,6 +204,8 @@ struct pd_sim {
   long partRows = 256;
   int partMax = 224;
   long partBodies = 96;     // bodies per workgroup, at least
+  int partAbsent = 0;       // tests: see PartSync
+  int partWaitPolls = PT_WAIT_POLLS;
   long partsBusy = 0;       // substeps to go before the partitioned loops are tried again ...
   long partsBusyNext = 64;  // ... after one found the device busy
   // extra slots reserved by setPositions for periodic ghosts (more are added when needed)
@@ -974,6 +976,11 @@ struct pd_sim {
     hNumPairs = -1;  // particle indices changed: the Hertz pair cache is stale, :1294-1295
     candForget();
     hPrevCount = 0;
+    if (stateLost) {  // the impulses and grounded levels of the failed substep go with it
+      prevCount = 0;
+      zero(ground.p, ground.cap);
+      stateLost = false;
+    }
     std::vector<double4> P((size_t)n);
     std::vector<BodyC> B((size_t)n);
     std::vector<Body64> V((size_t)n);
@@ -2030,6 +2037,8 @@ struct pd_sim {
     Y.over = ctl.p + CTL_PARTS_OVER;
     Y.fail = ctl.p + CTL_PARTS_FAIL;
     Y.refuse = refuse ? 1 : 0;
+    Y.absent = partAbsent;
+    Y.waitPolls = partWaitPolls;
     return Y;
   }
   bool vFusedRec = false;  // the timed K_VBLOCK record covers both loops of the stage
@@ -2110,7 +2119,15 @@ struct pd_sim {
   long sideStreamMinContacts = 0;
   // the adjoint replays each substep of a checkpoint segment once, into workspaces of its own
   bool adjKeepSegment = true;
+  // a substep failed after it had written velocities and impulses
+  bool stateLost = false;
+  void requireState() const {
+    if (stateLost)
+      throw std::runtime_error(
+          "the state was lost in a failed substep: set the positions and what goes with them");
+  }
   void demStep() {
+    requireState();
     std::memset(&stats, 0, sizeof stats);
     vbActive = nullptr;  // a substep cut short by an error may have left the stage's records
     vBlockRec[0] = vBlockRec[1] = pBlockRec = -1;
@@ -2802,8 +2819,10 @@ struct pd_sim {
         stats.stab_ran = usePGS ? c[CTL_STAB_RUN] : 0;
       }
       if (useGS && posLeftover == 0) posSweepsPrev = stats.sweeps_pos = c[CTL_SWEEPS_P];
-      if (c[CTL_PARTS_FAIL])
+      if (c[CTL_PARTS_FAIL]) {
+        stateLost = true;
         throw std::runtime_error("sweep loop: a workgroup waited too long for another");
+      }
       // a partitioned loop that found the device busy ran in one workgroup, slowly: the launches
       // per colour take over for a while, longer each time
       if (partsBusy > 0) {
@@ -2972,6 +2991,7 @@ struct pd_sim {
   }
   // demStepHertz, src/sim.hpp:628-750
   void stepHertz(double dtH, int nsteps, double skinFrac) {
+    requireState();
     dt = dtH;
     if (per[0] || per[1] || per[2])
       throw std::runtime_error("step_hertz: periodic domains not supported");
@@ -4157,6 +4177,13 @@ int pd_set_tuning(pd_sim* s, const char* name, long value) {
       if (value < 1 || value > PT_MAX_PARTS)
         throw ArgError("partition_workgroups must be in [1, " + std::to_string(PT_MAX_PARTS) + "]");
       s->partMax = (int)value;
+    } else if (k == "partition_absent") {
+      if (value != 0 && value != 2) throw ArgError("partition_absent must be 0 or 2");
+      s->partAbsent = (int)value;
+    } else if (k == "partition_wait_polls") {
+      if (value < 128 || value > PT_WAIT_POLLS)
+        throw ArgError("partition_wait_polls must be in [128, " + std::to_string(PT_WAIT_POLLS) + "]");
+      s->partWaitPolls = (int)value;
     } else if (k == "candidate_skin_permille") {
       if (value < 0) throw ArgError("candidate_skin_permille must be >= 0");
       s->candSkinFrac = std::min<long>(value, 100000) / 1000.0;

@@ -47,6 +47,50 @@ def test_partition_options(hip_lib, over):
     run_pair("bed_periodic", 400, 10, tuning={"partition_rows": 60}, **over)
 
 
+def set_state(sim, scene):
+    sim.set_positions(scene["pos"])
+    sim.set_scales(scene["scale"])
+    sim.set_inv_mass(scene["inv_mass"])
+    sim.set_inv_inertia(scene["inv_inertia"])
+    sim.set_velocities(scene["vel"])
+    sim.set_angular_velocities(scene["angvel"])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("loop", ["velocity", "position"])
+def test_a_wait_that_runs_out_fails_the_handle_until_it_is_set_again(hip_lib, loop):
+    # one workgroup leaves after the check-in, the others' waits run out: the step raises, the
+    # handle refuses to go on from the half-updated state, and a new state steps like a new handle
+    from peclet.dem import Simulation
+    from scenes import apply_scene, make_scene
+
+    scene = make_scene("bed_periodic", 400, 2)
+    scene["vel"][:, 2] -= 0.5
+    h = apply_scene(Simulation(400), scene)
+    h.set_tuning("partition_rows", 20)
+    h.set_tuning("velocity_loop_lds", 1 if loop == "velocity" else 0)
+    for _ in range(4):
+        h.step(scene["dt"])
+    assert h.get_stats()["sweeps_pos"] > 2
+    h.set_tuning("partition_wait_polls", 256)
+    h.set_tuning("partition_absent", 2)
+    with pytest.raises(RuntimeError, match="waited too long"):
+        h.step(scene["dt"])
+    h.set_tuning("partition_absent", 0)
+    for step in (h.step, lambda dt: h.step_n(dt, 2), lambda dt: h.step_hertz(dt, 1)):
+        with pytest.raises(RuntimeError, match="state was lost"):
+            step(scene["dt"])
+    set_state(h, scene)
+    other = apply_scene(Simulation(400), scene)
+    for _ in range(4):
+        h.step(scene["dt"])
+        other.step(scene["dt"])
+    for name in ("get_positions", "get_velocities", "get_angular_velocities"):
+        assert np.array_equal(getattr(h, name)(), getattr(other, name)()), name
+    h.close()
+    other.close()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind,n,tunings", [
     # enough rows for more than a hundred workgroups of several chunks per colour
