@@ -139,7 +139,12 @@ int pd_get_ledger(pd_sim* s, uint64_t* keys, double* lambda, double* lambdaT, do
 int pd_get_grounded(pd_sim* s, int* out, int n);
 /* how often each of the internal forms of a substep's parts was taken since the handle was made
  * (no reference counterpart): candidate pair list rebuilt, reused, left out for the substep;
- * returns the number of counters and writes at most cap of them */
+ * velocity loops over a partition, in one workgroup with the bodies in LDS, in one from global
+ * memory, in launches per colour; position loops likewise; loops of these with the last contact
+ * class as a chain, and the other classes over a partition beside it; partitioned loops whose
+ * check-in was refused and that became launches per colour, or ran in one workgroup; loops whose
+ * parts had more bodies than LDS slots.
+ * Returns the number of counters and writes at most cap of them */
 int pd_get_path_counts(pd_sim* s, long* out, int cap);
 
 /* --- host-side export ------------------------------------------------------------------- */
@@ -258,14 +263,16 @@ int pd_set_timing(pd_sim* s, int level);
  * stands for all that fit; the others stay in global memory), 0 leaves it to the one-workgroup
  * loop and the launches per colour; a "velocity_loop_lds_keys" below its default and maximum
  * 12288 makes a loop whose rows may have more distinct bodies leave that launch at its check-in
- * (one workgroup then runs the loop from global memory); "partition_rows" (default 256; 0 off,
+ * (one workgroup then runs the loop from global memory, or, above block_solver_rows rows, it
+ * becomes launches per colour); "partition_rows" (default 256; 0 off,
  * as is block_solver_rows 0): the rows per workgroup of the partitioned velocity and position
  * loops, four times as many for a loop in one workgroup; "partition_workgroups" (default 224, at
- * most 256): the most workgroups of one, "partition_bodies" (default 96): the fewest bodies per
+ * most 256; the default is less where the device has fewer than 256 compute units): the most
+ * workgroups of one, "partition_bodies" (default 96): the fewest bodies per
  * workgroup; "partition_wait_polls" (default and maximum 2^22, at least 128): the polls after which
  * a workgroup gives up waiting for another's body states, upon which the step fails and the handle
  * steps again only after pd_set_positions; "partition_absent" = 2 (default 0) makes one workgroup
- * leave them waiting, for tests of that; "vsweep_waves" = 3 (default)
+ * leave them waiting, 1 keep away from the check-in, for tests of either; "vsweep_waves" = 3 (default)
  * or 4 selects the per-colour PGS sweep compiled for that many waves per SIMD (4: at most 128
  * VGPRs, with some register spilling); "velocity_pack_bodies" = 1 (default) lets the per-colour
  * velocity launches read each body's velocity and constants from one 128-byte record packed for

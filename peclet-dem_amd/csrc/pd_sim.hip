@@ -206,8 +206,18 @@ struct pd_sim {
   long partBodies = 96;     // bodies per workgroup, at least
   int partAbsent = 0;       // tests: see PartSync
   int partWaitPolls = PT_WAIT_POLLS;
-  long partsBusy = 0;       // substeps to go before the partitioned loops are tried again ...
-  long partsBusyNext = 64;  // ... after one found the device busy
+  // substeps to go before the partitioned loops are tried again after one found the device busy;
+  // how many it will be the next time (doubled each time, halved after as many that ran); substeps
+  // whose loops ran since
+  static constexpr long BUSY_MIN = 64, BUSY_MAX = 4096;
+  long partsBusy = 0, partsBusyNext = BUSY_MIN, partsRan = 0;
+  bool partsRefused = false;  // a loop of this substep was refused
+  // how often each form of the sweep loops was taken (pd_get_path_counts)
+  struct Paths {
+    long velParts = 0, velOne = 0, velBlock = 0, velColours = 0;
+    long posParts = 0, posOne = 0, posBlock = 0, posColours = 0, chain = 0, chainParts = 0;
+    long refused = 0, alone = 0, global = 0;
+  } paths;
   // extra slots reserved by setPositions for periodic ghosts (more are added when needed)
   long slotHeadroom = 4096;
   // the largest scale, cached while no scale is written (every writer clears scaleKnown)
@@ -385,6 +395,10 @@ struct pd_sim {
     HIPCHECK(hipHostMalloc(&hostPost, 1024, hipHostMallocDefault));
     std::memset(hostPost, 0, 1024);
     HIPCHECK(hipHostGetDevicePointer(&hostPostDev, hostPost, 0));
+    int dev = 0, cus = 0;
+    HIPCHECK(hipGetDevice(&dev));
+    HIPCHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    partMax = std::max(1, std::min(partMax, cus * 7 / 8));  // (one workgroup per compute unit)
     HIPCHECK(hipHostGetDevicePointer(&jobV.pinnedDev, jobV.pinned, 0));
     HIPCHECK(hipHostGetDevicePointer(&jobP.pinnedDev, jobP.pinned, 0));
     jobV.stream = st;
@@ -508,9 +522,13 @@ struct pd_sim {
   // ~2 ms of waiting, since the runtime call takes locks that the other threads of a batch need
   // for their launches.
   static void waitPosted(const volatile int* seqp, int seq, hipStream_t s) {
+    waitUntil([=] { return *seqp == seq; }, s);
+  }
+  template <class F>
+  static void waitUntil(F&& posted, hipStream_t s) {
     auto last = std::chrono::steady_clock::now();
     for (long spin = 1;; ++spin) {
-      if (*seqp == seq) break;
+      if (posted()) break;
       __builtin_ia32_pause();
       if ((spin & 1023) == 0) {
         const auto now = std::chrono::steady_clock::now();
@@ -518,7 +536,7 @@ struct pd_sim {
         last = now;
         const hipError_t e = hipStreamQuery(s);
         if (e == hipSuccess) {
-          if (*seqp == seq) break;
+          if (posted()) break;
           throw std::runtime_error("read-back: the stream finished without posting");
         }
         if (e != hipErrorNotReady) HIPCHECK(e);
@@ -1912,11 +1930,13 @@ struct pd_sim {
     bool global = false;    // a part may have more bodies than LDS slots
     bool everOver = false;  // one had, unexpectedly
     PartList Q{};
+    int word;               // the check-in's outcome in the pinned area (64-bit words)
+    explicit PartJob(int w) : word(w) {}
     void release() {
       mem.release(); lines.release(); sync.release();
     }
   };
-  PartJob partsV, partsP;
+  PartJob partsV{64}, partsP{65};
   // from this many rows on the contact class 62 is run as a chain rather than by one thread
   static constexpr int CHAIN_MIN = 64;
   // the contact class 62 as a chain (k_psweep_chain): steps (first entry, rows) and entries
@@ -2016,7 +2036,8 @@ struct pd_sim {
     HIPCHECK(hipGetLastError());
   }
   // the exchange areas for a launch of at most `passes` passes
-  PartSync partSync(PartJob& J, int rows, int nd, long passes, bool refuse) {
+  // (`ask`: the host waits for the check-in, partsGo)
+  PartSync partSync(PartJob& J, int rows, int nd, long passes, bool refuse, bool ask) {
     PartSync Y{};
     if (J.seq > 0xFFFFFFFFu - (unsigned long)passes - 2 || J.epoch >= 0x7FFFFFFEu) {
       // the numbers start over: no line may hold an old one
@@ -2039,7 +2060,19 @@ struct pd_sim {
     Y.refuse = refuse ? 1 : 0;
     Y.absent = partAbsent;
     Y.waitPolls = partWaitPolls;
+    if (ask && J.Q.numParts > 1)
+      Y.outcome = static_cast<unsigned long long*>(hostPostDev) + J.word;
     return Y;
+  }
+  // the loop just launched runs (it was not asked, or all its workgroups checked in)
+  bool partsGo(const PartJob& J, const PartSync& Y) {
+    if (!Y.outcome) return true;
+    const volatile unsigned long long* w = static_cast<unsigned long long*>(hostPost) + J.word;
+    waitUntil([=] { return *w >> 1 == Y.epoch; }, st);
+    if (*w & 1u) return true;
+    partsRefused = true;
+    ++paths.refused;
+    return false;
   }
   bool vFusedRec = false;  // the timed K_VBLOCK record covers both loops of the stage
   long vBlockRec[2] = {-1, -1}, pBlockRec = -1;
@@ -2134,6 +2167,7 @@ struct pd_sim {
     sweepRecs.clear();
     curSweepTag = -1;
     vFusedRec = false;
+    partsRefused = false;
     timedNow = timing > 0 && timingSubstep % timingEvery == 0;
     ++timingSubstep;
     // a frictional wall drives friction even for frictionless bodies (src/sim.hpp:169-170)
@@ -2396,14 +2430,23 @@ struct pd_sim {
     }
     // the per-colour launches of a large bed read each row's bodies from one 128-byte record
     // per body, written by the predict launch or packed here, and unpacked when the stage ends
-    const bool usePack = packBodies && !hostLoop && !fusedV && !smallV && nRowsV > 0 &&
-                         numReal > 0 && (usePGS || velIters > 0);
-    if (usePack) {
-      vbody.ensure(numReal, st);
-      if (!vbFromPredict) k_vb_pack<<<nblk(numReal), TPB, 0, st>>>(dD, vbody.p, numReal);
-      vbActive = vbody.p;
-    }
-    vbUsedLast = usePack;
+    const bool usePack = packBodies && !hostLoop && !smallV && nRowsV > 0 && numReal > 0 &&
+                         (usePGS || velIters > 0);
+    vbUsedLast = false;
+    // the records, and the warm start of any other form than the one launch
+    auto warmStart = [&]() {
+      if (usePack) {
+        vbody.ensure(numReal, st);
+        if (!vbFromPredict) k_vb_pack<<<nblk(numReal), TPB, 0, st>>>(dD, vbody.p, numReal);
+        vbActive = vbody.p;
+      }
+      vbUsedLast = usePack;
+      if (!usePGS) return;
+      if (nRowsV <= blockRows)
+        vLoop(0, P, vs, numColors, 1, 0.0, 0.0, ctl.p + CTL_NONE, ctl.p + CTL_NONE, nullptr);
+      else
+        velocitySweep(vs, numColors, 0, 0.0, ctl.p + CTL_NONE);
+    };
     if (usePGS) {
       // grounded levels, double-buffered (src/contact_preprocessing.hpp:213-253); the decay ran
       // in the predict launch
@@ -2421,15 +2464,11 @@ struct pd_sim {
         }
       }
       // 8 swaps: the result is back in `ground`
-      if (!fusedV) {
-        if (nRowsV <= blockRows)
-          vLoop(0, P, vs, numColors, 1, 0.0, 0.0, ctl.p + CTL_NONE, ctl.p + CTL_NONE, nullptr);
-        else
-          velocitySweep(vs, numColors, 0, 0.0, ctl.p + CTL_NONE);
-      }
     }
+    if (!fusedV) warmStart();
     HIPCHECK(hipGetLastError());
     mark(ST_VSWEEP);
+    bool fusedRan = false;
     if (fusedV) {
       // warm start, sweep loop, stabilization gate, side flags and stabilization loop in one
       // launch
@@ -2454,17 +2493,31 @@ struct pd_sim {
       const int cap = ldsBodies < LDS_BODIES_MAX ? ldsBodies : PT_VBODIES;
       buildParts<true>(partsV, vAB.p, posPred.p, numReal, nRowsV, cs, numColors, cap);
       const PartSync Y = partSync(partsV, nRowsV, 6, 3L * velIters + 4,
-                                  ldsKeys < LDS_KEYS_MAX && 2L * nRowsV > ldsKeys);
+                                  ldsKeys < LDS_KEYS_MAX && 2L * nRowsV > ldsKeys, !smallV);
       const PartList& Q = partsV.Q;
       kernBegin();
       auto* const kernel = usePGS ? (partsV.global ? &k_vsolve_lds<1, true> : &k_vsolve_lds<1, false>)
                                   : (partsV.global ? &k_vsolve_lds<2, true> : &k_vsolve_lds<2, false>);
       kernel<<<Q.numParts, PT_V_THREADS, partLdsBytes(Q.cap, Q.numColors, 6), st>>>(dD, P, cs, S, Q, Y);
-      vBlockRec[0] = kernEnd(K_VBLOCK, nRowsV);
-      vFusedRec = true;
+      const long rec = kernEnd(K_VBLOCK, nRowsV);
       HIPCHECK(hipGetLastError());
+      // (the host would do this next: not held back by its wait)
+      if (Y.outcome && colourP && !colourPStarted) startContactColouring();
+      fusedRan = partsGo(partsV, Y);
+      if (fusedRan) {
+        vBlockRec[0] = rec;
+        vFusedRec = true;
+        ++(Q.numParts > 1 ? paths.velParts : paths.velOne);
+        paths.global += partsV.global ? 1 : 0;
+      } else {
+        if (rec >= 0) kernPending[rec].units = 0;
+        warmStart();
+      }
+    }
+    if (fusedRan) {
       mark(ST_STAB);
     } else if (!hostLoop) {
+      ++(smallV ? paths.velBlock : paths.velColours);
       // device-controlled adaptive stops: no host round trip per sweep
       const double stopThr = usePGS ? 0.02 * vRest : vRest;
       if (smallV && velIters > 0) {
@@ -2643,13 +2696,36 @@ struct pd_sim {
     const int rows62 = numPosColors == 63 ? ps[63] - ps[62] : 0;
     const bool chainFits = rows62 >= CHAIN_MIN && partRows > 0 && blockRows > 0 &&
                            numParticles <= CHAIN_SLOTS;
-    const bool posBatches = useGS && posLeftover == 0 && (nRowsP > blockRows || chainFits) && !posParts;
+    // (what a partitioned loop of more than blockRows rows becomes when it is refused)
+    const bool posBatches = useGS && posLeftover == 0 && (nRowsP > blockRows || chainFits);
     if (nRowsP > 0)
       k_prows<<<nblk(nc), TPB, 0, st>>>(dD, nc, posBatches ? bits.p : nullptr);
     mark(ST_PSWEEP);
     const double posTol = 1e-4 * baseRadius * globalScale;
     const int* finalCtl = nullptr;
     const unsigned long long* finalBits = nullptr;
+    bool posRan = false;
+    if (posParts) {
+      const ClassStarts pcs = classStarts(ps);
+      buildParts<false>(partsP, pAB.p, posPred.p, numParticles, nRowsP, pcs, numPosColors,
+                        PT_PBODIES);
+      const PartSync Y = partSync(partsP, nRowsP, 3, posIters + 1L, false, posBatches);
+      const PartList& Q = partsP.Q;
+      kernBegin();
+      auto* const kernel = partsP.global ? &k_psolve_lds<true> : &k_psolve_lds<false>;
+      kernel<<<Q.numParts, PT_P_THREADS, partLdsBytes(Q.cap, Q.numColors, 3), st>>>(
+          dD, pcs, posIters, posTol, ctl.p + CTL_STOP_P, ctl.p + CTL_SWEEPS_P, Q, Y, nullptr);
+      const long rec = kernEnd(K_PBLOCK, nRowsP);
+      HIPCHECK(hipGetLastError());
+      posRan = partsGo(partsP, Y);
+      if (posRan) {
+        pBlockRec = rec;
+        ++(Q.numParts > 1 ? paths.posParts : paths.posOne);
+        paths.global += partsP.global ? 1 : 0;
+      } else if (rec >= 0) {
+        kernPending[rec].units = 0;
+      }
+    }
     if (!useGS) {
       // Jacobi XPBD over every contact, no adaptive stop (src/solver_position.hpp:34-134)
       if (posIters > 0) buildIncidence<1>(nc, 0);
@@ -2658,20 +2734,10 @@ struct pd_sim {
         stats.sweeps_pos++;
       }
       HIPCHECK(hipGetLastError());
-    } else if (posParts) {
-      const ClassStarts pcs = classStarts(ps);
-      buildParts<false>(partsP, pAB.p, posPred.p, numParticles, nRowsP, pcs, numPosColors,
-                        PT_PBODIES);
-      const PartSync Y = partSync(partsP, nRowsP, 3, posIters + 1L, false);
-      const PartList& Q = partsP.Q;
-      kernBegin();
-      auto* const kernel = partsP.global ? &k_psolve_lds<true> : &k_psolve_lds<false>;
-      kernel<<<Q.numParts, PT_P_THREADS, partLdsBytes(Q.cap, Q.numColors, 3), st>>>(
-          dD, pcs, posIters, posTol, ctl.p + CTL_STOP_P, ctl.p + CTL_SWEEPS_P, Q, Y, nullptr);
-      pBlockRec = kernEnd(K_PBLOCK, nRowsP);
-      HIPCHECK(hipGetLastError());
+    } else if (posRan) {
     } else if (posLeftover == 0 && !posBatches) {
       if (posIters > 0) {
+        ++paths.posBlock;
         kernBegin();
         k_psolve_block<<<1, BLOCK_SOLVER_THREADS, 0, st>>>(dD, classStarts(ps), numPosColors,
                                                            posIters, posTol, ctl.p + CTL_STOP_P,
@@ -2723,20 +2789,26 @@ struct pd_sim {
       }
       // beside a chain, the other classes of a sweep run in one launch over a partition (3,001
       // packed rings, 62 classes: 257 us per sweep in a launch each, 170 us in one)
-      const bool partSweeps = chain > 0 && partsTake(ps[62], 62, 3, 1L << 30);
+      bool partSweeps = chain > 0 && partsTake(ps[62], 62, 3, 1L << 30);
       if (partSweeps)
         buildParts<false>(partsP, pAB.p, posPred.p, numParticles, ps[62], pcs, 62, PT_PBODIES);
+      ++paths.posColours;
+      paths.chain += chain > 0 ? 1 : 0;
+      paths.chainParts += partSweeps ? 1 : 0;
       int done = 0, batch = std::max(1, std::min(posIters, posSweepsPrev));
       // (the residual was cleared by the rows launch)
       while (done < posIters) {
         const int b = std::min(batch, posIters - done);
         for (int j = 0; j < b; ++j) {
           if (partSweeps) {
-            const PartSync Y = partSync(partsP, ps[62], 3, 2, false);
+            // (asked once: a refusal of a later sweep keeps the rest from the check-in)
+            const PartSync Y = partSync(partsP, ps[62], 3, 2, false, done + j == 0);
             const PartList& Q = partsP.Q;
             auto* const kernel = partsP.global ? &k_psolve_lds<true> : &k_psolve_lds<false>;
             kernel<<<Q.numParts, PT_P_THREADS, partLdsBytes(Q.cap, Q.numColors, 3), st>>>(
                 dD, pcs, 1, -1.0, ctl.p + CTL_DUMP, ctl.p + CTL_DUMP, Q, Y, ctl.p + CTL_STOP_P);
+            HIPCHECK(hipGetLastError());
+            partSweeps = partsGo(partsP, Y);  // (refused: launches from here on)
           }
           for (int c = partSweeps ? 62 : 0; c < cFrom; ++c) {
             const int cb = ps[c], ce = ps[c + 1];
@@ -2823,15 +2895,20 @@ struct pd_sim {
         stateLost = true;
         throw std::runtime_error("sweep loop: a workgroup waited too long for another");
       }
-      // a partitioned loop that found the device busy ran in one workgroup, slowly: the launches
-      // per colour take over for a while, longer each time
+      // a partitioned loop that found the device busy cost its check-in: the other forms take over
+      // for a while
+      paths.alone += c[CTL_PARTS_BUSY] ? 1 : 0;
       if (partsBusy > 0) {
         --partsBusy;
       } else if (c[CTL_PARTS_OVER]) {
         partsV.everOver = partsP.everOver = true;
-      } else if (c[CTL_PARTS_BUSY] && ldsKeys == LDS_KEYS_MAX) {
+      } else if ((c[CTL_PARTS_BUSY] || partsRefused) && ldsKeys == LDS_KEYS_MAX) {
         partsBusy = partsBusyNext;
-        partsBusyNext = std::min(4096L, 2 * partsBusyNext);
+        partsBusyNext = std::min(BUSY_MAX, 2 * partsBusyNext);
+        partsRan = 0;
+      } else if (partsBusyNext > BUSY_MIN && (fusedRan || posRan) && ++partsRan >= partsBusyNext) {
+        partsBusyNext /= 2;
+        partsRan = 0;
       }
       maxOverlap = bitsd(b2[0]);
       maxApproach = bitsd(b2[1]);
@@ -3993,7 +4070,10 @@ int pd_get_ledger(pd_sim* s, uint64_t* keys, double* lambda, double* lambdaT, do
   return s->prevCount;
 }
 int pd_get_path_counts(pd_sim* s, long* out, int cap) {
-  const long v[] = {s->candRebuilds, s->candReuses, s->candSkipped};
+  const auto& p = s->paths;
+  const long v[] = {s->candRebuilds, s->candReuses, s->candSkipped, p.velParts, p.velOne,
+                    p.velBlock, p.velColours, p.posParts, p.posOne, p.posBlock, p.posColours,
+                    p.chain, p.chainParts, p.refused, p.alone, p.global};
   const int n = (int)(sizeof(v) / sizeof(v[0]));
   for (int k = 0; out && k < n && k < cap; ++k) out[k] = v[k];
   return n;
@@ -4178,7 +4258,7 @@ int pd_set_tuning(pd_sim* s, const char* name, long value) {
         throw ArgError("partition_workgroups must be in [1, " + std::to_string(PT_MAX_PARTS) + "]");
       s->partMax = (int)value;
     } else if (k == "partition_absent") {
-      if (value != 0 && value != 2) throw ArgError("partition_absent must be 0 or 2");
+      if (value < 0 || value > 2) throw ArgError("partition_absent must be 0, 1 or 2");
       s->partAbsent = (int)value;
     } else if (k == "partition_wait_polls") {
       if (value < 128 || value > PT_WAIT_POLLS)

@@ -615,7 +615,10 @@ class Simulation:
         self._b.get_grounded(self._h, out.ctypes.data_as(C.POINTER(C.c_int)), n)
         return out
 
-    PATHS = ("list_rebuilt", "list_reused", "list_left_out")
+    PATHS = ("list_rebuilt", "list_reused", "list_left_out",
+             "vel_parts", "vel_one", "vel_block", "vel_colours",
+             "pos_parts", "pos_one", "pos_block", "pos_colours", "chain", "chain_parts",
+             "refused", "alone", "global")
 
     def debug_paths(self):
         """How often each internal form of a substep's parts was taken (extension)."""

@@ -47,6 +47,87 @@ def test_partition_options(hip_lib, over):
     run_pair("bed_periodic", 400, 10, tuning={"partition_rows": 60}, **over)
 
 
+def bodies(sim):
+    return [sim.get_positions(), sim.get_velocities(), sim.get_angular_velocities(),
+            *sim.debug_ledger()]
+
+
+def assert_same_bodies(a, b, tag):
+    for k, (x, y) in enumerate(zip(bodies(a), bodies(b))):
+        assert np.array_equal(x, y), (tag, k)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("block_rows", [16384, 100], ids=["alone", "launches"])
+def test_check_in_that_times_out(hip_lib, block_rows):
+    # one workgroup keeps away: the others agree to leave, and the loop runs in one workgroup, or,
+    # above block_solver_rows rows, in launches per colour; the partition is then left alone for 64
+    # substeps
+    from peclet.dem import Simulation
+    from scenes import apply_scene, make_scene
+
+    scene = make_scene("bed_periodic", 1500, 2)
+    scene["vel"][:, 2] -= 0.5
+    h, plain = (apply_scene(Simulation(1500), scene) for _ in range(2))
+    plain.set_tuning("block_solver_rows", 0)
+    h.set_tuning("partition_rows", 20)
+    h.set_tuning("block_solver_rows", block_rows)
+    h.set_tuning("partition_absent", 1)
+    for k in range(3):
+        h.step(scene["dt"])
+        plain.step(scene["dt"])
+        assert h.get_stats() == plain.get_stats()
+        assert_same_bodies(h, plain, k)
+    paths = h.debug_paths()
+    assert (paths["alone"], paths["refused"]) == ((1, 0) if block_rows == 16384 else (0, 1))
+    assert paths["vel_parts"] == (1 if block_rows == 16384 else 0)
+    h.set_tuning("partition_absent", 0)
+    h.step_n(scene["dt"], 62)
+    plain.step_n(scene["dt"], 62)
+    assert h.debug_paths()["vel_parts"] == paths["vel_parts"]
+    h.step_n(scene["dt"], 4)
+    plain.step_n(scene["dt"], 4)
+    after = h.debug_paths()
+    print(paths, after, flush=True)
+    assert after["vel_parts"] == paths["vel_parts"] + 4 and after["refused"] == paths["refused"]
+    assert_same_bodies(h, plain, "after")
+    h.close()
+    plain.close()
+
+
+@pytest.mark.gpu
+def test_two_large_systems_at_once(hip_lib):
+    # each takes more than half of the compute units: loops that cannot have all their workgroups
+    # running become launches per colour, and either system's states are those of a run by itself
+    import threading
+
+    from peclet.dem import Simulation
+    from scenes import apply_scene, make_scene
+
+    n, steps = 90000, 12
+    scenes = [make_scene("bed_periodic", n, seed) for seed in (1, 2)]
+    alone = []
+    for sc in scenes:
+        h = apply_scene(Simulation(n), sc)
+        h.step_n(sc["dt"], steps)
+        alone.append(bodies(h))
+        h.close()
+    pair = [apply_scene(Simulation(n), sc) for sc in scenes]
+    threads = [threading.Thread(target=h.step_n, args=(sc["dt"], steps))
+               for h, sc in zip(pair, scenes)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for h, want in zip(pair, alone):
+        paths = h.debug_paths()
+        print(paths, flush=True)
+        assert paths["alone"] == 0 and paths["vel_parts"] + paths["vel_colours"] == steps
+        for x, y in zip(bodies(h), want):
+            assert np.array_equal(x, y)
+        h.close()
+
+
 def set_state(sim, scene):
     sim.set_positions(scene["pos"])
     sim.set_scales(scene["scale"])
@@ -118,8 +199,10 @@ def test_partition_equals_the_launches_per_colour(hip_lib, kind, n, tunings):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tuning", [{}, {"partition_bodies": 20}, {"partition_rows": 0}],
-                         ids=["chain", "more-parts", "launches"])
+@pytest.mark.parametrize("tuning", [{}, {"partition_bodies": 20},
+                                    {"partition_bodies": 20, "partition_absent": 1},
+                                    {"partition_rows": 0}],
+                         ids=["chain", "more-parts", "refused", "launches"])
 def test_last_contact_class_as_a_chain(hip_lib, tuning):
     # packed hollow cylinders with a dense shell: hundreds of rows in the contact class whose rows
     # share bodies, walked by one wavefront beside the other classes' partition, or in launches
@@ -143,6 +226,15 @@ def test_last_contact_class_as_a_chain(hip_lib, tuning):
         colours = h.debug_contact_colors()
         assert np.array_equal(colours, r.debug_contact_colors())
     assert (colours == 62).sum() > 64
+    paths = h.debug_paths()
+    if "partition_rows" in tuning:
+        assert paths["chain"] == 0 and paths["chain_parts"] == 0
+    else:
+        assert paths["chain"] == 2
+        # (a refusal in the first substep's first sweep keeps the second substep off the partition)
+        absent = "partition_absent" in tuning
+        assert paths["chain_parts"] == (1 if absent else 2)
+        assert paths["refused"] == (1 if absent else 0) and paths["alone"] == 0
 
 
 @pytest.mark.gpu
