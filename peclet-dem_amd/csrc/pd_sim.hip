@@ -989,10 +989,14 @@ struct pd_sim {
     // headroom for the periodic ghosts (src/periodicity.hpp:25-38); grown on demand
     const long est = (long)n + (long)n / 4 + slotHeadroom;
     ensureSlots((int)std::max<long>(est, capacity), numReal);
+    const int was = numReal;
     numReal = n;
     numParticles = n;
     hNumPairs = -1;  // particle indices changed: the Hertz pair cache is stale, :1294-1295
-    candForget();
+    // (a system put back where it was keeps what its lists have shown: 3,001 rings put back every
+    // two substeps, 19.6 ms against 19.8 ms)
+    candValid = false;
+    if (n != was) candForget();
     hPrevCount = 0;
     if (stateLost) {  // the impulses and grounded levels of the failed substep go with it
       prevCount = 0;
@@ -1109,7 +1113,7 @@ struct pd_sim {
   int candFails = 0;
   long candSkip = 0, candSkipped = 0;
   static constexpr long CAND_SKIP_MAX = 64;
-  // a new skin or new positions: neither the list nor what its predecessors did says anything
+  // a new skin or other bodies: neither the list nor what its predecessors did says anything
   void candForget() {
     candValid = false;
     candReused = true;
