@@ -140,7 +140,8 @@ int pd_get_grounded(pd_sim* s, int* out, int n);
 /* how often each of the internal forms of a substep's parts was taken since the handle was made
  * (no reference counterpart): candidate pair list rebuilt, reused, left out for the substep;
  * velocity loops over a partition, in one workgroup with the bodies in LDS, in one from global
- * memory, in launches per colour; position loops likewise; loops of these with the last contact
+ * memory, in launches per colour; position loops over a partition, in one workgroup from global
+ * memory, in launches per colour; loops of these last with the last contact
  * class as a chain, and the other classes over a partition beside it; partitioned loops whose
  * check-in was refused and that became launches per colour, or ran in one workgroup; loops whose
  * parts had more bodies than LDS slots.
@@ -266,7 +267,8 @@ int pd_set_timing(pd_sim* s, int level);
  * (one workgroup then runs the loop from global memory, or, above block_solver_rows rows, it
  * becomes launches per colour); "partition_rows" (default 256; 0 off,
  * as is block_solver_rows 0): the rows per workgroup of the partitioned velocity and position
- * loops, four times as many for a loop in one workgroup; "partition_workgroups" (default 224, at
+ * loops, four times as many for a velocity loop in one workgroup; position loops are partitioned
+ * from twenty times as many on; "partition_workgroups" (default 224, at
  * most 256; the default is less where the device has fewer than 256 compute units): the most
  * workgroups of one, "partition_bodies" (default 96): the fewest bodies per
  * workgroup; "partition_wait_polls" (default and maximum 2^22, at least 128): the polls after which

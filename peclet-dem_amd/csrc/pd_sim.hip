@@ -215,7 +215,7 @@ struct pd_sim {
   // how often each form of the sweep loops was taken (pd_get_path_counts)
   struct Paths {
     long velParts = 0, velOne = 0, velBlock = 0, velColours = 0;
-    long posParts = 0, posOne = 0, posBlock = 0, posColours = 0, chain = 0, chainParts = 0;
+    long posParts = 0, posBlock = 0, posColours = 0, chain = 0, chainParts = 0;
     long refused = 0, alone = 0, global = 0;
   } paths;
   // extra slots reserved by setPositions for periodic ghosts (more are added when needed)
@@ -1948,6 +1948,11 @@ struct pd_sim {
   DBuf<int4> chainEnt;
   std::vector<int2> chainStepsHost;
   static constexpr long PT_SINGLE = 4;
+  // Position rows: up to this many times partRows the loop of one workgroup reading positions
+  // through its L1 is the shorter one, having less to do per colour (12 sweeps of 9 colours, one
+  // workgroup / partition: 1,475 rows 131 / 229 us, 4,491 rows 208 / 242, 6,337 rows 342 / 260,
+  // 12,463 rows 618 / 265; 12 of 54 colours, 739 rows: 461 / 923)
+  static constexpr long PT_POS_MIN = 20;
   static constexpr size_t PT_LINE_BYTES_MAX = 0xFFFFFF00u;  // (32-bit line offsets)
   // The partitioned loop takes rows whose classes leave out the last one (62, whose rows may share
   // a body), up to maxRows of them.
@@ -2695,7 +2700,8 @@ struct pd_sim {
     refreshDev();
     // with the batched position loop ahead, the rows launch also clears its residual
     // (a loop that stops after a sweep or two does not repay building a partition)
-    const bool posParts = useGS && posLeftover == 0 && posIters > 0 && nRowsP > 0 &&
+    const bool posParts = useGS && posLeftover == 0 && posIters > 0 &&
+                          nRowsP > PT_POS_MIN * partRows && numParticles >= partBodies &&
                           posSweepsPrev > 2 && partsTake(nRowsP, numPosColors, 3, 1L << 30);
     const int rows62 = numPosColors == 63 ? ps[63] - ps[62] : 0;
     const bool chainFits = rows62 >= CHAIN_MIN && partRows > 0 && blockRows > 0 &&
@@ -2724,7 +2730,7 @@ struct pd_sim {
       posRan = partsGo(partsP, Y);
       if (posRan) {
         pBlockRec = rec;
-        ++(Q.numParts > 1 ? paths.posParts : paths.posOne);
+        ++paths.posParts;
         paths.global += partsP.global ? 1 : 0;
       } else if (rec >= 0) {
         kernPending[rec].units = 0;
@@ -4076,7 +4082,7 @@ int pd_get_ledger(pd_sim* s, uint64_t* keys, double* lambda, double* lambdaT, do
 int pd_get_path_counts(pd_sim* s, long* out, int cap) {
   const auto& p = s->paths;
   const long v[] = {s->candRebuilds, s->candReuses, s->candSkipped, p.velParts, p.velOne,
-                    p.velBlock, p.velColours, p.posParts, p.posOne, p.posBlock, p.posColours,
+                    p.velBlock, p.velColours, p.posParts, p.posBlock, p.posColours,
                     p.chain, p.chainParts, p.refused, p.alone, p.global};
   const int n = (int)(sizeof(v) / sizeof(v[0]));
   for (int k = 0; out && k < n && k < cap; ++k) out[k] = v[k];

@@ -617,7 +617,7 @@ class Simulation:
 
     PATHS = ("list_rebuilt", "list_reused", "list_left_out",
              "vel_parts", "vel_one", "vel_block", "vel_colours",
-             "pos_parts", "pos_one", "pos_block", "pos_colours", "chain", "chain_parts",
+             "pos_parts", "pos_block", "pos_colours", "chain", "chain_parts",
              "refused", "alone", "global")
 
     def debug_paths(self):

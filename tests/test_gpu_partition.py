@@ -96,6 +96,28 @@ def test_check_in_that_times_out(hip_lib, block_rows):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind,n,form", [("bed_walls", 500, "pos_block"),
+                                         ("big_among_small", 600, "pos_block"),
+                                         ("bed_walls", 4000, "pos_parts")])
+def test_form_of_the_position_loop(hip_lib, kind, n, form):
+    # loops of fewer than 5,120 rows run in one workgroup from global memory, the form that is the
+    # shorter one there
+    from peclet.dem import Simulation
+    from scenes import apply_scene, make_scene
+
+    scene = make_scene(kind, n, 5)
+    h = apply_scene(Simulation(len(scene["pos"])), scene)
+    h.step_n(scene["dt"], 12)
+    before = h.debug_paths()
+    h.step_n(scene["dt"], 8)
+    after = h.debug_paths()
+    print(kind, n, h.get_stats()["num_contacts"], before, after, flush=True)
+    assert h.get_stats()["sweeps_pos"] > 2
+    assert after[form] == before[form] + 8
+    h.close()
+
+
+@pytest.mark.gpu
 def test_two_large_systems_at_once(hip_lib):
     # each takes more than half of the compute units: loops that cannot have all their workgroups
     # running become launches per colour, and either system's states are those of a run by itself
