@@ -1941,8 +1941,15 @@ struct pd_sim {
     }
   };
   PartJob partsV{64}, partsP{65};
-  // from this many rows on the contact class 62 is run as a chain rather than by one thread
-  static constexpr int CHAIN_MIN = 64;
+  // from this many rows on the contact class 62 is run as a chain rather than by one thread; in a
+  // loop that one workgroup could run, where the chain costs the host a read-back, launches and its
+  // order, only from CHAIN_MIN_SMALL rows on and where they are not the rows of one or two large
+  // bodies, hardly more than one to a step (the class before it has CHAIN_WIDTH rows).  ms per
+  // substep in one workgroup / with the chain: 201 spheres, one touching all, 138 rows, width 1:
+  // 0.95 / 1.12; 4,630 slots around a sphere of ten radii, 270 rows, width 1: 9.0 / 10.4; 216
+  // boxes, 5-77 rows, width 2-6: 1.86 / 2.24; 100 rings, 830-1,160 rows, width 21-41: 11.1 / 8.3;
+  // 512 boxes, 1,440-1,910 rows, width 46-81: 10.2 / 4.8
+  static constexpr int CHAIN_MIN = 64, CHAIN_MIN_SMALL = 512, CHAIN_WIDTH = 8;
   // the contact class 62 as a chain (k_psweep_chain): steps (first entry, rows) and entries
   DBuf<int2> chainSteps;
   DBuf<int4> chainEnt;
@@ -2704,7 +2711,10 @@ struct pd_sim {
                           nRowsP > PT_POS_MIN * partRows && numParticles >= partBodies &&
                           posSweepsPrev > 2 && partsTake(nRowsP, numPosColors, 3, 1L << 30);
     const int rows62 = numPosColors == 63 ? ps[63] - ps[62] : 0;
-    const bool chainFits = rows62 >= CHAIN_MIN && partRows > 0 && blockRows > 0 &&
+    const bool chainGains = nRowsP > blockRows ? rows62 >= CHAIN_MIN
+                                               : rows62 >= CHAIN_MIN_SMALL &&
+                                                     ps[62] - ps[61] >= CHAIN_WIDTH;
+    const bool chainFits = chainGains && partRows > 0 && blockRows > 0 &&
                            numParticles <= CHAIN_SLOTS;
     // (what a partitioned loop of more than blockRows rows becomes when it is refused)
     const bool posBatches = useGS && posLeftover == 0 && (nRowsP > blockRows || chainFits);
