@@ -208,8 +208,9 @@ struct pd_sim {
   int partWaitPolls = PT_WAIT_POLLS;
   // substeps to go before the partitioned loops are tried again after one found the device busy;
   // how many it will be the next time (doubled each time, halved after as many that ran); substeps
-  // whose loops ran since
-  static constexpr long BUSY_MIN = 64, BUSY_MAX = 4096;
+  // whose loops ran since.  (A refused check-in costs 2 ms and the loop's other form, and each
+  // substep without the partition 0.4 to 2.3 ms: 1,000 to 4,000 spheres 1.24 / 1.61, 1.59 / 3.91 ms)
+  static constexpr long BUSY_MIN = 4, BUSY_MAX = 4096;
   long partsBusy = 0, partsBusyNext = BUSY_MIN, partsRan = 0;
   bool partsRefused = false;  // a loop of this substep was refused
   // how often each form of the sweep loops was taken (pd_get_path_counts)
@@ -1964,8 +1965,9 @@ struct pd_sim {
   // The partitioned loop takes rows whose classes leave out the last one (62, whose rows may share
   // a body), up to maxRows of them.
   bool partsTake(int rows, int numColors, int nd, long maxRows) const {
-    return partRows > 0 && blockRows > 0 && partsBusy == 0 && numColors <= PT_COLORS &&
-           rows <= maxRows && (size_t)rows * 4 * 16 * nd <= PT_LINE_BYTES_MAX;
+    return partRows > 0 && blockRows > 0 &&
+           (partsBusy == 0 || rows <= PT_SINGLE * partRows) &&  // (no check-in in one workgroup)
+           numColors <= PT_COLORS && rows <= maxRows && (size_t)rows * 4 * 16 * nd <= PT_LINE_BYTES_MAX;
   }
   // Velocity rows: above this many the launches per colour move their rows faster than 224
   // workgroups whose bodies no longer all fit in LDS (ms per substep, launches / partition: 0.55M

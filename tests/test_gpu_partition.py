@@ -61,7 +61,7 @@ def assert_same_bodies(a, b, tag):
 @pytest.mark.parametrize("block_rows", [16384, 100], ids=["alone", "launches"])
 def test_check_in_that_times_out(hip_lib, block_rows):
     # one workgroup keeps away: the others agree to leave, and the loop runs in one workgroup, or,
-    # above block_solver_rows rows, in launches per colour; the partition is then left alone for 64
+    # above block_solver_rows rows, in launches per colour; the partition is then left alone for 4
     # substeps
     from peclet.dem import Simulation
     from scenes import apply_scene, make_scene
@@ -82,14 +82,14 @@ def test_check_in_that_times_out(hip_lib, block_rows):
     assert (paths["alone"], paths["refused"]) == ((1, 0) if block_rows == 16384 else (0, 1))
     assert paths["vel_parts"] == (1 if block_rows == 16384 else 0)
     h.set_tuning("partition_absent", 0)
-    h.step_n(scene["dt"], 62)
-    plain.step_n(scene["dt"], 62)
+    h.step_n(scene["dt"], 2)
+    plain.step_n(scene["dt"], 2)
     assert h.debug_paths()["vel_parts"] == paths["vel_parts"]
-    h.step_n(scene["dt"], 4)
-    plain.step_n(scene["dt"], 4)
+    h.step_n(scene["dt"], 10)
+    plain.step_n(scene["dt"], 10)
     after = h.debug_paths()
     print(paths, after, flush=True)
-    assert after["vel_parts"] == paths["vel_parts"] + 4 and after["refused"] == paths["refused"]
+    assert after["vel_parts"] == paths["vel_parts"] + 10 and after["refused"] == paths["refused"]
     assert_same_bodies(h, plain, "after")
     h.close()
     plain.close()
