@@ -110,7 +110,8 @@ struct PartSync {
   unsigned seq0;     // passes of this launch are numbered seq0 + 1, ...
   unsigned epoch;
   int* busy;         // set when one workgroup ran the loop alone: no more check-ins this substep
-  int* over;         // set when a part had more bodies than LDS slots
+  int* over;         // gets overBit when a part had more bodies than LDS slots
+  int overBit;       // (1: velocity rows, 2: position rows)
   int* fail;         // set when a wait ran out
   // where the outcome of the check-in goes in host memory, epoch << 1 | 1 for all running: then
   // nobody runs the loop alone (null: workgroup 0 does)
@@ -1108,7 +1109,7 @@ __global__ __launch_bounds__(PT_V_THREADS) void k_vsolve_lds(const Dev* __restri
   if (parts == 1) partSingle(Q, D.vAB, cs, table);
   const bool fits = GLOB || Q.partCnt[me] <= Q.cap;
   if (!partCheckIn(Y, me, parts, fits, &go)) {
-    if (tid == 0 && !fits) stDevice(Y.over, 1);
+    if (tid == 0 && !fits) atomicOr(Y.over, Y.overBit);
     if (me != 0 || Y.outcome) return;
     if (tid == 0) *Y.busy = 1;
     vStageAlone<MODE>(D, P, cs, Q.numColors, S, sh);
@@ -1260,7 +1261,7 @@ __global__ __launch_bounds__(PT_P_THREADS) void k_psolve_lds(const Dev* __restri
   if (parts == 1) partSingle(Q, D.pAB, cs, table);
   const bool fits = GLOB || Q.partCnt[me] <= Q.cap;
   if (!partCheckIn(Y, me, parts, fits, &go)) {
-    if (tid == 0 && !fits) stDevice(Y.over, 1);
+    if (tid == 0 && !fits) atomicOr(Y.over, Y.overBit);
     if (me != 0 || Y.outcome) return;
     if (tid == 0) *Y.busy = 1;
     pSweepLoop(D, cs, Q.numColors, iters, tol, stop, count, sh);

@@ -213,6 +213,7 @@ struct pd_sim {
   static constexpr long BUSY_MIN = 4, BUSY_MAX = 4096;
   long partsBusy = 0, partsBusyNext = BUSY_MIN, partsRan = 0;
   bool partsRefused = false;  // a loop of this substep was refused
+  static constexpr long OVER_LOOPS = 64;
   // how often each form of the sweep loops was taken (pd_get_path_counts)
   struct Paths {
     long velParts = 0, velOne = 0, velBlock = 0, velColours = 0;
@@ -1932,8 +1933,8 @@ struct pd_sim {
     DBuf<pu4> lines;
     DBuf<pu4> sync;           // maxima [2 x PT_MAX_PARTS], then the check-ins and the decision
     unsigned seq = 0, epoch = 0;
-    bool global = false;    // a part may have more bodies than LDS slots
-    bool everOver = false;  // one had, unexpectedly
+    bool global = false;  // a part may have more bodies than LDS slots
+    long overFor = 0;     // one had, unexpectedly: loops to go with it expected
     PartList Q{};
     int word;               // the check-in's outcome in the pinned area (64-bit words)
     explicit PartJob(int w) : word(w) {}
@@ -1993,10 +1994,17 @@ struct pd_sim {
                                                 (rows + partRows - 1) / partRows);
     const int levels = partLevels(parts), cells = parts > 1 ? 1 << levels : 0;
     const long most = std::min<long>(ids, 2L * rows);
-    // (a part's bodies number at most about 1.7 times the average: k_part_hist's weights)
-    const long room = 2 * ((most + parts - 1) / parts) + 64;
-    const int capL = (int)std::min<long>(cap, room);
-    J.global = room > cap || J.everOver;
+    // A body weighs its rows and two more (k_part_hist), so a part whose bodies have one row each
+    // holds a third of its share of the weight, many times the average number of bodies where the
+    // others have many rows: LDS slots for that many, and a quarter more for cells cut unevenly.
+    // (Which of the kernels runs is decided by twice the average: the other one costs the loops
+    // that would have fitted.)
+    const long share = (2L * rows + 2 * most + 3 * parts - 1) / (3 * parts);
+    const long twice = 2 * ((most + parts - 1) / parts) + 64;
+    const int capL =
+        (int)std::min<long>(cap, std::min<long>(most, std::max(twice, share + share / 4 + 64)));
+    J.global = twice > cap || J.overFor > 0;
+    if (J.overFor > 0) --J.overFor;
     const int bkts = parts * std::max(1, numColors);
     const long entries = (parts > 1 ? 2L : 1L) * rows + (long)PT_CHUNK * bkts;
     PartList& Q = J.Q;
@@ -2074,6 +2082,7 @@ struct pd_sim {
     Y.epoch = ++J.epoch;
     Y.busy = ctl.p + CTL_PARTS_BUSY;
     Y.over = ctl.p + CTL_PARTS_OVER;
+    Y.overBit = &J == &partsV ? 1 : 2;
     Y.fail = ctl.p + CTL_PARTS_FAIL;
     Y.refuse = refuse ? 1 : 0;
     Y.absent = partAbsent;
@@ -2923,7 +2932,8 @@ struct pd_sim {
       if (partsBusy > 0) {
         --partsBusy;
       } else if (c[CTL_PARTS_OVER]) {
-        partsV.everOver = partsP.everOver = true;
+        if (c[CTL_PARTS_OVER] & 1) partsV.overFor = OVER_LOOPS;
+        if (c[CTL_PARTS_OVER] & 2) partsP.overFor = OVER_LOOPS;
       } else if ((c[CTL_PARTS_BUSY] || partsRefused) && ldsKeys == LDS_KEYS_MAX) {
         partsBusy = partsBusyNext;
         partsBusyNext = std::min(BUSY_MAX, 2 * partsBusyNext);

@@ -122,6 +122,48 @@ def test_form_of_the_position_loop(hip_lib, kind, n, form):
 
 
 @pytest.mark.gpu
+def test_parts_of_bodies_with_one_row_each(hip_lib):
+    # a dense block (about 18 contacts a sphere) and as many spheres in pairs: a part of pairs holds
+    # several times the average number of bodies, and still has LDS slots for all of them
+    from peclet.dem import Simulation
+
+    r, rng = 1e-3, np.random.default_rng(4)
+    g = np.stack(np.meshgrid(*[np.arange(12)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    dense = (g + 1.0) * 1.4 * r + rng.uniform(-0.01, 0.01, g.shape) * r
+    m = np.stack(np.meshgrid(*[np.arange(10)] * 3, indexing="ij"), -1).reshape(-1, 3)[:864]
+    pairs = np.array([0.0, 0.0, 0.03]) + (m + 1.0) * 6.0 * r
+    pairs = np.concatenate([pairs, pairs + np.array([1.9 * r, 0.0, 0.0])])
+    pos = np.concatenate([dense, pairs])
+    n = len(pos)
+
+    def system(**tuning):
+        h = Simulation(n)
+        h.set_sphere_shape(r)
+        h.set_domain(0.08, 0.08, 0.12, False, False, False)
+        h.set_positions(pos)
+        h.set_velocities(np.random.default_rng(5).normal(0.0, 0.05, (n, 3)))
+        h.set_gravity(0.0, 0.0, -9.81)
+        h.set_material_params(0.3, 0.2, 0.5)
+        h.set_solver_iterations(6, 6)
+        for key, value in tuning.items():
+            h.set_tuning(key, value)
+        return h
+
+    h, plain = system(), system(block_solver_rows=0)
+    for k in range(4):
+        h.step(1e-5)
+        plain.step(1e-5)
+        assert h.get_stats() == plain.get_stats()
+        assert_same_bodies(h, plain, k)
+    paths = h.debug_paths()
+    print(h.get_stats(), paths, flush=True)
+    assert paths["vel_parts"] == 4 and paths["pos_parts"] == 3
+    assert (paths["alone"], paths["refused"], paths["global"]) == (0, 0, 0)
+    h.close()
+    plain.close()
+
+
+@pytest.mark.gpu
 def test_two_large_systems_at_once(hip_lib):
     # each takes more than half of the compute units: loops that cannot have all their workgroups
     # running become launches per colour, and either system's states are those of a run by itself
