@@ -83,6 +83,7 @@ struct PartList {
   int* listStart;  // [ids] where each id's rows start in list
   int* list;       // [2 x rows] each id's rows in colour order: 2 x row + side, sign bit: between
   int* listCnt;    // places of list given out
+  int* skew;       // set when one part holds far more rows than the others
   int* hist;       // [cells] weight
   int* cellStart;  // [cells + 1] its scan
   int* partOf;     // [ids] part << 20 | place in the part
@@ -163,20 +164,81 @@ __device__ __forceinline__ int partCell(const PartGrid& g, double4 p) {
   }
   return code;
 }
-// clears the counters; thread 0 lays the cells over the broadphase grid's box
-__global__ void k_part_begin(PartList Q, const Grid* box, int ids, int cells, int levels) {
+// The extent of the rows' bodies, from 16 x 16 rows spread evenly, one per thread: the medians of
+// the 16 groups' smallest and largest coordinates, about the 4 % and 96 % quantiles.  A few bodies
+// far away (one that left its container) do not move them.  What is no number is left as it was.
+__device__ __forceinline__ void partExtent(const double (&x)[3], double* lo, double* hi) {
+  __shared__ double sh[6][16];
+  double a[3], b[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    a[d] = b[d] = x[d];
+    for (int off = 1; off < 16; off <<= 1) {
+      a[d] = fmin(a[d], __shfl_xor(a[d], off, 64));
+      b[d] = fmax(b[d], __shfl_xor(b[d], off, 64));
+    }
+    if ((threadIdx.x & 15) == 0) {
+      sh[d][threadIdx.x >> 4] = a[d];
+      sh[3 + d][threadIdx.x >> 4] = b[d];
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < 96) {
+    const int q = (int)threadIdx.x >> 4, me = (int)threadIdx.x & 15;
+    const double own = sh[q][me];
+    int rank = 0;
+    for (int j = 0; j < 16; ++j) {
+      const double v = sh[q][j];
+      rank += v < own || (v == own && j < me) ? 1 : 0;
+    }
+    if (q < 3 && rank == 7) lo[q] = own;
+    if (q >= 3 && rank == 8) hi[q - 3] = own;
+  }
+  __syncthreads();
+}
+// Clears the counters; the first workgroup lays the cells over the rows' bodies: over the
+// quantiles above and 0.15 of their distance on either side, within the broadphase grid's box (the
+// halvings are few, and would be spent on the way to one distant body: 9,001 spheres, one a
+// thousand bed widths away: 1.26 ms of velocity loops against 0.36).  Bodies outside fall into the
+// outermost cells.
+__global__ __launch_bounds__(TPB) void k_part_begin(PartList Q, const Grid* box, const int2* ends,
+                                                    const double4* pos, int ids, int rows, int cells,
+                                                    int levels) {
+  static_assert(TPB == 256, "16 groups of 16 samples");
   const int i = gtid();
   if (i < ids) Q.mask[i] = 0ull;
   if (i == 0) *Q.listCnt = 0;
   if (i < cells) Q.hist[i] = 0;
   if (i < Q.numParts) Q.partCnt[i] = 0;
   if (i < Q.numParts * Q.numColors * 2) Q.bktCnt[i] = 0;
+  if (blockIdx.x != 0) return;
+  __shared__ double lo[3], hi[3];
+  const Grid b = *box;
+  const double e[3] = {b.h * b.dim[0], b.h * b.dim[1], b.h * b.dim[2]};
+  const double boxLo[3] = {b.lo.x, b.lo.y, b.lo.z};
+  if (i < 3) {
+    lo[i] = boxLo[i];
+    hi[i] = boxLo[i] + e[i];
+  }
+  const int sample = ((int)threadIdx.x & 15) * 16 + ((int)threadIdx.x >> 4);
+  const double4 p = pos[ends[(int)((long)sample * rows / TPB)].x];
+  const double xyz[3] = {p.x, p.y, p.z};
+  partExtent(xyz, lo, hi);
   if (i == 0) {
     PartGrid g;
-    const Grid b = *box;
-    double ex = b.h * b.dim[0], ey = b.h * b.dim[1], ez = b.h * b.dim[2];
+    double l[3], w[3];
+    for (int d = 0; d < 3; ++d) {
+      const double m = 0.15 * (hi[d] - lo[d]);
+      l[d] = fmax(lo[d] - m, boxLo[d]);
+      w[d] = fmin(hi[d] + m, boxLo[d] + e[d]) - l[d];
+      if (!(w[d] > 0.0)) {
+        l[d] = boxLo[d];
+        w[d] = e[d];
+      }
+    }
+    double ex = w[0], ey = w[1], ez = w[2];
     int dx = 1, dy = 1, dz = 1;
-    g.lo = b.lo;
+    g.lo = d3{l[0], l[1], l[2]};
     g.levels = levels;
     g.axes = 0;
     for (int l = 0; l < levels; ++l) {
@@ -313,9 +375,11 @@ __global__ __launch_bounds__(1024) void k_part_count(PartList Q, const int2* end
   }
   Q.rank[k] = r;
 }
-// entry ranges: every (part, colour) starts a new chunk.  One workgroup.
-__global__ __launch_bounds__(1024) void k_part_ranges(PartList Q) {
-  __shared__ int waveTot[16];
+// entry ranges: every (part, colour) starts a new chunk.  One workgroup.  A part that holds
+// several times the average and more than its workgroup takes at once (`wide` rows of every colour)
+// keeps all others waiting: bodies in places far apart, which the cells did not separate.
+__global__ __launch_bounds__(1024) void k_part_ranges(PartList Q, int wide) {
+  __shared__ int waveTot[16], first[PT_MAX_PARTS + 1];
   const int n = Q.numParts * Q.numColors;
   const int per = (n + 1023) / 1024;
   const int b0 = (int)threadIdx.x * per, e0 = min(b0 + per, n);
@@ -333,9 +397,19 @@ __global__ __launch_bounds__(1024) void k_part_ranges(PartList Q) {
   for (int w = 0; w < wave; ++w) at += waveTot[w];
   for (int i = b0; i < e0; ++i) {
     const int nb = Q.bktCnt[2 * i], ni = Q.bktCnt[2 * i + 1];
+    if (i % Q.numColors == 0) first[i / Q.numColors] = at;
     Q.bkt[i] = make_int4(at, nb, nb + ni, 0);
     at += (nb + ni + PT_CHUNK - 1) & ~(PT_CHUNK - 1);
+    if (i == n - 1) first[Q.numParts] = at;
   }
+  __syncthreads();
+  bool uneven = false;
+  if ((int)threadIdx.x < Q.numParts) {
+    const long own = first[threadIdx.x + 1] - first[threadIdx.x];
+    uneven = own * Q.numParts > 4L * first[Q.numParts] && own > (long)wide * Q.numColors;
+  }
+  const int any = __syncthreads_or(uneven ? 1 : 0);
+  if (threadIdx.x == 0) *Q.skew = any;
 }
 // VEL: also the second copies of the impulses and flags of the rows between parts
 template <bool VEL>
@@ -1107,8 +1181,9 @@ __global__ __launch_bounds__(PT_V_THREADS) void k_vsolve_lds(const Dev* __restri
   double* const body = reinterpret_cast<double*>(ptBody);
   int4* const table = reinterpret_cast<int4*>(ptBody + (Q.cap * 6 + 1) / 2);
   if (parts == 1) partSingle(Q, D.vAB, cs, table);
-  const bool fits = GLOB || Q.partCnt[me] <= Q.cap;
-  if (!partCheckIn(Y, me, parts, fits, &go)) {
+  const bool even = parts == 1 || *Q.skew == 0;
+  const bool fits = !even || GLOB || Q.partCnt[me] <= Q.cap;
+  if (!partCheckIn(Y, me, parts, even && fits, &go)) {
     if (tid == 0 && !fits) atomicOr(Y.over, Y.overBit);
     if (me != 0 || Y.outcome) return;
     if (tid == 0) *Y.busy = 1;
@@ -1259,8 +1334,9 @@ __global__ __launch_bounds__(PT_P_THREADS) void k_psolve_lds(const Dev* __restri
   double* const body = reinterpret_cast<double*>(ptBody);
   int4* const table = reinterpret_cast<int4*>(ptBody + (Q.cap * 3 + 1) / 2);
   if (parts == 1) partSingle(Q, D.pAB, cs, table);
-  const bool fits = GLOB || Q.partCnt[me] <= Q.cap;
-  if (!partCheckIn(Y, me, parts, fits, &go)) {
+  const bool even = parts == 1 || *Q.skew == 0;
+  const bool fits = !even || GLOB || Q.partCnt[me] <= Q.cap;
+  if (!partCheckIn(Y, me, parts, even && fits, &go)) {
     if (tid == 0 && !fits) atomicOr(Y.over, Y.overBit);
     if (me != 0 || Y.outcome) return;
     if (tid == 0) *Y.busy = 1;

@@ -1996,13 +1996,14 @@ struct pd_sim {
     const long most = std::min<long>(ids, 2L * rows);
     // A body weighs its rows and two more (k_part_hist), so a part whose bodies have one row each
     // holds a third of its share of the weight, many times the average number of bodies where the
-    // others have many rows: LDS slots for that many, and a quarter more for cells cut unevenly.
+    // others have many rows: LDS slots for that many, and a quarter more for cells cut unevenly,
+    // and for as many as take half of the LDS in any case.
     // (Which of the kernels runs is decided by twice the average: the other one costs the loops
     // that would have fitted.)
     const long share = (2L * rows + 2 * most + 3 * parts - 1) / (3 * parts);
     const long twice = 2 * ((most + parts - 1) / parts) + 64;
     const int capL =
-        (int)std::min<long>(cap, std::min<long>(most, std::max(twice, share + share / 4 + 64)));
+        (int)std::min<long>(cap, std::min(most, std::max({twice, share + share / 4 + 64, cap / 2L})));
     J.global = twice > cap || J.overFor > 0;
     if (J.overFor > 0) --J.overFor;
     const int bkts = parts * std::max(1, numColors);
@@ -2021,7 +2022,7 @@ struct pd_sim {
         off += (n * sizeof(T) + 255) & ~(size_t)255;
       };
       take(Q.partOf, ids + 1);
-      take(Q.partCnt, PT_MAX_PARTS + 1);  // (and the lists' counter)
+      take(Q.partCnt, PT_MAX_PARTS + 2);  // (and the lists' counter, and skew)
       take(Q.partIds, (size_t)parts * capL);
       take(Q.bktCnt, 2 * bkts);
       take(Q.bkt, bkts);
@@ -2046,17 +2047,18 @@ struct pd_sim {
     J.mem.ensure(lay(nullptr), st);
     lay(J.mem.p);
     Q.listCnt = Q.partCnt + PT_MAX_PARTS;
+    Q.skew = Q.listCnt + 1;
     J.sync.ensure(2 * PT_MAX_PARTS + (PT_MAX_PARTS + 1 + 3) / 4, st);
     if (parts > 1) J.lines.ensure((size_t)rows * 4 * (VEL ? 6 : 3), st);
     if (parts > 1) {  // (a loop of one workgroup builds its partition itself)
       k_part_begin<<<nblk(std::max(std::max(ids, cells), 2 * bkts)), TPB, 0, st>>>(
-          Q, gridD.p, ids, cells, levels);
+          Q, gridD.p, ends, posOf, ids, rows, cells, levels);
       k_part_colours<<<nblk(rows), TPB, 0, st>>>(Q, ends, cs, rows);
       k_part_hist<<<nblk(ids), TPB, 0, st>>>(Q, posOf, ids);
       scanQuiet(Q.hist, Q.cellStart, cells);
       k_part_assign<<<(ids + 1023) / 1024, 1024, 0, st>>>(Q, posOf, ids, cells);
       k_part_count<<<(rows + 1023) / 1024, 1024, 0, st>>>(Q, ends, cs, rows);
-      k_part_ranges<<<1, 1024, 0, st>>>(Q);
+      k_part_ranges<<<1, 1024, 0, st>>>(Q, (VEL ? PT_V_THREADS : PT_P_THREADS) / 2);
       k_part_fill<VEL><<<nblk(rows), TPB, 0, st>>>(dD, Q, ends, cs, rows);
     }
     HIPCHECK(hipGetLastError());
@@ -2926,14 +2928,13 @@ struct pd_sim {
         stateLost = true;
         throw std::runtime_error("sweep loop: a workgroup waited too long for another");
       }
-      // a partitioned loop that found the device busy cost its check-in: the other forms take over
-      // for a while
+      // a partitioned loop that found the device busy, its parts uneven or too large cost its
+      // check-in: the other forms take over for a while
       paths.alone += c[CTL_PARTS_BUSY] ? 1 : 0;
+      if (c[CTL_PARTS_OVER] & 1) partsV.overFor = OVER_LOOPS;
+      if (c[CTL_PARTS_OVER] & 2) partsP.overFor = OVER_LOOPS;
       if (partsBusy > 0) {
         --partsBusy;
-      } else if (c[CTL_PARTS_OVER]) {
-        if (c[CTL_PARTS_OVER] & 1) partsV.overFor = OVER_LOOPS;
-        if (c[CTL_PARTS_OVER] & 2) partsP.overFor = OVER_LOOPS;
       } else if ((c[CTL_PARTS_BUSY] || partsRefused) && ldsKeys == LDS_KEYS_MAX) {
         partsBusy = partsBusyNext;
         partsBusyNext = std::min(BUSY_MAX, 2 * partsBusyNext);

@@ -122,6 +122,42 @@ def test_form_of_the_position_loop(hip_lib, kind, n, form):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("block_rows", [16384, 1000])
+@pytest.mark.parametrize("far", ["one-body", "half"])
+def test_bodies_far_apart(hip_lib, far, block_rows):
+    # a sphere a thousand bed widths from its bed: the partition is that of the bed.  Two beds as far
+    # from each other: a few parts hold all rows, which the loops notice before they start
+    from peclet.dem import Simulation
+    from scenes import apply_scene, make_scene
+
+    n = 9000
+    scene = make_scene("bed", n, 5)
+    width = scene["domain"][0]
+    if far == "one-body":
+        scene["pos"][-1] = [1000.0 * width, 0.5 * width, 0.02]
+    else:
+        scene["pos"][n // 2:] = scene["pos"][:n - n // 2] + np.array([1000.0 * width, 0.0, 0.0])
+    h, plain = (apply_scene(Simulation(n), scene) for _ in range(2))
+    plain.set_tuning("block_solver_rows", 0)
+    h.set_tuning("block_solver_rows", block_rows)
+    for k in range(3):
+        h.step(scene["dt"])
+        plain.step(scene["dt"])
+        assert h.get_stats() == plain.get_stats()
+        assert_same_bodies(h, plain, k)
+    paths = h.debug_paths()
+    print(far, h.get_stats(), paths, flush=True)
+    if far == "one-body":
+        assert (paths["vel_parts"], paths["alone"], paths["refused"]) == (3, 0, 0)
+    else:
+        # (the loops of one substep, then the pause)
+        assert 1 <= paths["alone"] + paths["refused"] <= 2
+        assert block_rows == 16384 or paths["alone"] == 0
+    h.close()
+    plain.close()
+
+
+@pytest.mark.gpu
 def test_parts_of_bodies_with_one_row_each(hip_lib):
     # a dense block (about 18 contacts a sphere) and as many spheres in pairs: a part of pairs holds
     # several times the average number of bodies, and still has LDS slots for all of them
