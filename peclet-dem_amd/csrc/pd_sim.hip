@@ -1962,18 +1962,25 @@ struct pd_sim {
   // workgroup / partition: 1,475 rows 131 / 229 us, 4,491 rows 208 / 242, 6,337 rows 342 / 260,
   // 12,463 rows 618 / 265; 12 of 54 colours, 739 rows: 461 / 923)
   static constexpr long PT_POS_MIN = 20;
-  static constexpr size_t PT_LINE_BYTES_MAX = 0xFFFFFF00u;  // (32-bit line offsets)
   // The partitioned loop takes rows whose classes leave out the last one (62, whose rows may share
   // a body), up to maxRows of them.
-  bool partsTake(int rows, int numColors, int nd, long maxRows) const {
+  bool partsTake(int rows, int numColors, long maxRows) const {
     return partRows > 0 && blockRows > 0 &&
            (partsBusy == 0 || rows <= PT_SINGLE * partRows) &&  // (no check-in in one workgroup)
-           numColors <= PT_COLORS && rows <= maxRows && (size_t)rows * 4 * 16 * nd <= PT_LINE_BYTES_MAX;
+           numColors <= PT_COLORS && rows <= maxRows;
   }
   // Velocity rows: above this many the launches per colour move their rows faster than 224
-  // workgroups whose bodies no longer all fit in LDS (ms per substep, launches / partition: 0.55M
-  // rows of a 1M pour 6.79 / 6.28, 1.96M rows of a resting 1M bed 16.0 / 17.0).
-  static constexpr long PARTS_V_ROWS = 1L << 20;
+  // workgroups whose bodies no longer all fit in LDS (ms of velocity loops per substep of a resting
+  // bed, launches / partition: 0.45M rows 2.54 / 2.13, 0.93M 4.00 / 3.79, 1.05M 4.24 / 4.41; ms per
+  // substep of 1M spheres, 1.96M rows 16.0 / 17.0).
+  static constexpr long PARTS_V_ROWS = 1000000;
+  // Position rows: the two forms are within a tenth of each other from half a million rows on, up
+  // to this many (ms of position loops per substep, launches / partition: 0.30M rows 0.52 / 0.46,
+  // 0.60M 0.69 / 0.72, 0.90M 0.90 / 0.88, 1.2M 1.04 / 1.18, 1.5M 1.35 / 1.33, 3.1M 2.71 / 2.62,
+  // 4.2M 3.37 / 3.35; 6M 4.73 / 5.54, 12M 8.98 / 12.94).
+  static constexpr long PARTS_P_ROWS = 1L << 22;
+  // (line offsets have 32 bits)
+  static_assert(PARTS_V_ROWS * 4 * 16 * 6 <= 0xFFFFFF00L && PARTS_P_ROWS * 4 * 16 * 3 <= 0xFFFFFF00L);
   static int partLevels(int parts) {  // about 64 cells per part
     int l = 6;
     while ((1 << l) < 64 * parts && (1 << l) < PT_MAX_CELLS) ++l;
@@ -2438,8 +2445,8 @@ struct pd_sim {
     // cylinders, 8.8M contacts and 0.52M rows, 47.8 ms against 4.4 ms by launches per colour,
     // about what one workgroup alone takes; 1M poured spheres, ~1M contacts and 0.55M rows, gain)
     const bool fusedV = !hostLoop && velIters > 0 && ldsLoop &&
-                        (nRowsV <= blockRows || nc <= 2 * PARTS_V_ROWS) &&
-                        partsTake(nRowsV, numColors, 6, PARTS_V_ROWS);
+                        (nRowsV <= blockRows || nc <= 1 << 21) &&
+                        partsTake(nRowsV, numColors, PARTS_V_ROWS);
     const size_t R = nRowsV + 1;
     vAB.ensure(R, st); vN.ensure(R, st); vTA.ensure(R, st); vTB.ensure(R, st); vRA.ensure(R, st);
     vRB.ensure(R, st); vVt0.ensure(R, st); vLamT.ensure(R, st); vVn0.ensure(R, st);
@@ -2722,7 +2729,7 @@ struct pd_sim {
     // (a loop that stops after a sweep or two does not repay building a partition)
     const bool posParts = useGS && posLeftover == 0 && posIters > 0 &&
                           nRowsP > PT_POS_MIN * partRows && numParticles >= partBodies &&
-                          posSweepsPrev > 2 && partsTake(nRowsP, numPosColors, 3, 1L << 30);
+                          posSweepsPrev > 2 && partsTake(nRowsP, numPosColors, PARTS_P_ROWS);
     const int rows62 = numPosColors == 63 ? ps[63] - ps[62] : 0;
     const bool chainGains = nRowsP > blockRows ? rows62 >= CHAIN_MIN
                                                : rows62 >= CHAIN_MIN_SMALL &&
@@ -2822,7 +2829,7 @@ struct pd_sim {
       }
       // beside a chain, the other classes of a sweep run in one launch over a partition (3,001
       // packed rings, 62 classes: 257 us per sweep in a launch each, 170 us in one)
-      bool partSweeps = chain > 0 && partsTake(ps[62], 62, 3, 1L << 30);
+      bool partSweeps = chain > 0 && partsTake(ps[62], 62, PARTS_P_ROWS);
       if (partSweeps)
         buildParts<false>(partsP, pAB.p, posPred.p, numParticles, ps[62], pcs, 62, PT_PBODIES);
       ++paths.posColours;

@@ -200,6 +200,23 @@ def test_parts_of_bodies_with_one_row_each(hip_lib):
 
 
 @pytest.mark.gpu
+def test_very_large_loops_are_launches_per_colour(hip_lib):
+    from peclet.dem import Simulation
+    from scenes import apply_scene, make_scene
+
+    n = 1600000
+    scene = make_scene("bed_periodic", n, 1)
+    h = apply_scene(Simulation(n), scene)
+    h.step_n(scene["dt"], 3)
+    paths, stats = h.debug_paths(), h.get_stats()
+    print(stats, paths, flush=True)
+    assert stats["active_manifolds"] > 1000000 and stats["num_contacts"] > 1 << 22
+    assert stats["sweeps_pos"] > 2
+    assert (paths["vel_colours"], paths["pos_colours"]) == (3, 3)
+    h.close()
+
+
+@pytest.mark.gpu
 def test_two_large_systems_at_once(hip_lib):
     # each takes more than half of the compute units: loops that cannot have all their workgroups
     # running become launches per colour, and either system's states are those of a run by itself
@@ -280,6 +297,8 @@ def test_a_wait_that_runs_out_fails_the_handle_until_it_is_set_again(hip_lib, lo
 @pytest.mark.parametrize("kind,n,tunings", [
     # enough rows for more than a hundred workgroups of several chunks per colour
     ("bed_periodic", 20000, [{}, {"partition_workgroups": 7}]),
+    # the most workgroups, of several times partition_rows rows each
+    ("bed_periodic", 140000, [{}]),
     # a sphere wider than its box: rows of a body and its own image
     ("big_among_small", 300, [{}, {"partition_rows": 10}])])
 def test_partition_equals_the_launches_per_colour(hip_lib, kind, n, tunings):
@@ -296,6 +315,14 @@ def test_partition_equals_the_launches_per_colour(hip_lib, kind, n, tunings):
         h.step_n(scene["dt"], 6)
         runs.append((h.get_positions(), h.get_velocities(), h.get_angular_velocities(),
                      *h.debug_ledger(), h.get_stats()))
+        paths = h.debug_paths()
+        print(paths, flush=True)
+        if "block_solver_rows" in tuning:
+            assert paths["vel_parts"] + paths["vel_one"] + paths["pos_parts"] == 0
+        else:
+            assert paths["vel_parts" if n > 1000 else "vel_one"] == 6
+            assert paths["pos_parts"] == (5 if n > 1000 or "partition_rows" in tuning else 0)
+            assert (paths["refused"], paths["alone"]) == (0, 0)
         h.close()
     for other in runs[1:]:
         for a, b in zip(runs[0], other):
