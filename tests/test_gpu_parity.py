@@ -128,10 +128,14 @@ def test_bed_periodic_multistep(hip_lib, block_rows):
                          ids=["global", "lds-and-global", "lds-fallback"])
 def test_velocity_loop_body_storage(hip_lib, kind, tuning):
     # the one-workgroup velocity loops default to bodies staged in LDS; here they keep them in
-    # global memory, or stage only 24 bodies and leave the rest in global memory, or give up
-    # staging above 16 distinct bodies (the gated global-memory loop then runs): every variant
-    # is the oracle's result
-    run_pair(kind, 300, 15, tuning=tuning)
+    # global memory, or stage only 24 bodies and leave the rest in global memory, or leave where
+    # the rows may have more than 16 distinct bodies (the same launch then runs the loop from
+    # global memory): every variant is the oracle's result
+    h, _ = run_pair(kind, 300, 15, tuning=tuning)
+    paths = h.debug_paths()
+    assert paths["vel_block" if "velocity_loop_lds" in tuning else "vel_one"] == 15
+    assert paths["global"] == (15 if "velocity_loop_lds_bodies" in tuning else 0)
+    assert (paths["alone"] > 0) == ("velocity_loop_lds_keys" in tuning)
 
 
 @pytest.mark.gpu
@@ -198,11 +202,11 @@ def test_sphere_in_shell_thousands_of_edges_at_one_body(hip_lib, tuning):
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,steps", [(2500, 4), (4000, 3)])
 def test_velocity_stage_large_beds(hip_lib, n, steps):
-    # 2500 spheres: ~4500-6700 rows over ~2900 bodies, so the staged stage keeps 2400 bodies in
-    # LDS and the rest in global memory, with several rounds per colour and the stabilization
-    # loop running; 4000 spheres: more than 8192 rows, so staging gives up and the gated
-    # global-memory launches run the stage
-    run_pair("bed_periodic", n, steps)
+    # 4500 to 10600 velocity rows and 7600 to 12200 position rows: both loops over a partition of 18
+    # to 42 workgroups, the stabilization loop running
+    h, _ = run_pair("bed_periodic", n, steps)
+    paths = h.debug_paths()
+    assert paths["vel_parts"] == steps and paths["pos_parts"] == steps - 1
 
 
 @pytest.mark.gpu

@@ -13,7 +13,17 @@ ROWS = [100000, 200, 33, 9]
 @pytest.mark.parametrize("kind", ["bed", "bed_periodic", "gas", "bed_walls"])
 @pytest.mark.parametrize("rows", ROWS)
 def test_partition_sizes(hip_lib, kind, rows):
-    run_pair(kind, 500, 12, tuning={"partition_rows": rows})
+    h, _ = run_pair(kind, 500, 12, tuning={"partition_rows": rows})
+    paths = h.debug_paths()
+    print(paths, flush=True)
+    assert paths["vel_parts"] + paths["vel_one"] == 12
+    assert (paths["refused"], paths["alone"], paths["global"]) == (0, 0, 0)
+    # (position loops: from 20 x rows on, after a loop of more than two sweeps; the gas thins out)
+    gas = kind == "gas"
+    vel, pos = {100000: (0, 0), 200: (0 if gas else 3, 0), 33: (1 if gas else 11, 0 if gas else 10),
+                9: (3 if gas else 12, 3 if gas else 10)}[rows]
+    assert paths["vel_parts"] >= vel and paths["pos_parts"] >= pos
+    assert vel or paths["vel_parts"] == 0
 
 
 @pytest.mark.gpu
@@ -24,7 +34,18 @@ def test_partition_sizes(hip_lib, kind, rows):
 def test_partition_shapes_and_twins(hip_lib, kind, n, steps, rows):
     # several points per manifold, every sphere with images of its neighbours, and (the big sphere)
     # colourings whose last class keeps the loops off the partition
-    run_pair(kind, n, steps, tuning={"partition_rows": rows})
+    h, _ = run_pair(kind, n, steps, tuning={"partition_rows": rows, "partition_bodies": 8})
+    paths = h.debug_paths()
+    print(paths, flush=True)
+    assert (paths["refused"], paths["alone"]) == (0, 0)
+    if kind == "big_among_small":
+        assert (paths["vel_parts"], paths["vel_block"], paths["pos_parts"]) == (2, 1, 0)
+    elif rows == 9:
+        assert paths["vel_parts"] >= (1 if kind in ("boxes", "cylinders") else steps)
+        # (the contacts of the cylinders are not all coloured)
+        assert paths["pos_parts"] >= {"cylinders": 0, "boxes": 1}.get(kind, steps - 1)
+    else:
+        assert paths["vel_one"] == steps
 
 
 @pytest.mark.gpu
@@ -35,7 +56,15 @@ def test_partition_shapes_and_twins(hip_lib, kind, n, steps, rows):
 def test_partition_storage_and_check_in(hip_lib, kind, tuning):
     # parts with more bodies than LDS slots; workgroups that agree to leave at the check-in, so that
     # one of them runs the loop; more rows per workgroup than asked for
-    run_pair(kind, 300, 10, tuning={"partition_rows": 20, **tuning})
+    h, _ = run_pair(kind, 300, 10, tuning={"partition_rows": 20, **tuning})
+    paths = h.debug_paths()
+    print(paths, flush=True)
+    assert paths["vel_parts"] >= (1 if kind == "gas" else 6)
+    assert paths["global"] == (10 if "velocity_loop_lds_bodies" in tuning else 0)
+    if "velocity_loop_lds_keys" in tuning:
+        assert paths["alone"] >= (3 if kind == "gas" else 10)
+    else:
+        assert paths["alone"] == 0
 
 
 @pytest.mark.gpu
@@ -44,7 +73,10 @@ def test_partition_storage_and_check_in(hip_lib, kind, tuning):
                          ids=["no-tangential", "frictionless", "no-stabilization", "one-sweep",
                               "no-position-loop"])
 def test_partition_options(hip_lib, over):
-    run_pair("bed_periodic", 400, 10, tuning={"partition_rows": 60}, **over)
+    h, _ = run_pair("bed_periodic", 400, 10, tuning={"partition_rows": 60}, **over)
+    paths = h.debug_paths()
+    # (a position loop of one sweep does not repay a partition)
+    assert paths["vel_parts"] == 10 and paths["pos_parts"] == (0 if "iters" in over else 9)
 
 
 def bodies(sim):
@@ -373,7 +405,10 @@ def test_last_contact_class_as_a_chain(hip_lib, tuning):
 def test_candidate_list_left_out_after_failures(hip_lib, skin):
     # images that come and go, and a skin that every step outruns: lists that fail at their first
     # reuse, the substeps that go without one, and the next list
-    run_pair("bed_periodic", 300, 50, tuning={"candidate_skin_permille": skin})
+    h, _ = run_pair("bed_periodic", 300, 50, tuning={"candidate_skin_permille": skin})
+    paths = h.debug_paths()
+    assert paths["list_rebuilt"] == 3 and paths["list_left_out"] >= 33
+    assert (paths["list_reused"] > 0) == (skin == 100)
 
 
 @pytest.mark.gpu
