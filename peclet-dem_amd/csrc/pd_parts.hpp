@@ -33,7 +33,8 @@
 // Waiting needs all workgroups to be running.  They first check in; if they are not all running
 // within a bounded time (other work holds the compute units) they agree, through one compare-and-
 // swap, to leave.  Workgroup 0 then runs a small loop alone from global memory; of a larger one the
-// host waits for the outcome of the check-in, and takes the launches per colour.  Once all have checked in
+// host waits for the outcome of the check-in, and takes the launches per colour.  They leave as well
+// where one part holds most of the rows or more bodies than LDS slots.  Once all have checked in
 // every wait ends, since a workgroup never leaves before the loop does; the waits are bounded all
 // the same, in polls and not by a clock (a process may be suspended for any time, and its polls
 // with it), and a wait that runs out raises an error on the host.
@@ -197,10 +198,10 @@ __device__ __forceinline__ void partExtent(const double (&x)[3], double* lo, dou
   __syncthreads();
 }
 // Clears the counters; the first workgroup lays the cells over the rows' bodies: over the
-// quantiles above and 0.15 of their distance on either side, within the broadphase grid's box (the
-// halvings are few, and would be spent on the way to one distant body: 9,001 spheres, one a
-// thousand bed widths away: 1.26 ms of velocity loops against 0.36).  Bodies outside fall into the
-// outermost cells.
+// quantiles above and 0.15 of their distance on either side, within the broadphase grid's box.
+// Bodies outside fall into the outermost cells.  (The halvings are few and would be spent on the
+// way to one distant body: with 9,001 spheres, one of them a thousand bed widths away, the velocity
+// loops took 1.26 ms over the whole box and take 0.36 over the quantiles.)
 __global__ __launch_bounds__(TPB) void k_part_begin(PartList Q, const Grid* box, const int2* ends,
                                                     const double4* pos, int ids, int rows, int cells,
                                                     int levels) {

@@ -190,13 +190,14 @@ struct pd_sim {
   HzDev Z{};
   // sweep loops over at most this many rows run in one workgroup (k_vsolve_block/k_psolve_block)
   int blockRows = BLOCK_SOLVER_ROWS;
-  bool ldsLoop = true;  // one-workgroup velocity loops stage their bodies in LDS when they fit
   bool vsweepWaves4 = false;  // per-colour PGS sweeps compiled for 4 waves per SIMD
-  // ... up to this many per workgroup (the rest stay in global memory; LDS_BODIES_MAX: all that fit)
+  // velocity loops run over a partition of the bodies, in one launch with the bodies in LDS, up to
+  // this many per workgroup (the rest stay in global memory; LDS_BODIES_MAX: all that fit)
+  bool ldsLoop = true;
   static constexpr int LDS_BODIES_MAX = 2400;
   int ldsBodies = LDS_BODIES_MAX;
-  // rows that may have more distinct bodies than this: the loop leaves at its check-in and one
-  // workgroup runs it from global memory (LDS_KEYS_MAX: never)
+  // rows that may have more distinct bodies than this: the loop leaves at its check-in
+  // (LDS_KEYS_MAX: never)
   static constexpr int LDS_KEYS_MAX = 12288;
   int ldsKeys = LDS_KEYS_MAX;
   // sweep loops over a partition of the bodies (pd_parts.hpp): rows per workgroup (0: off) and the
@@ -1992,9 +1993,9 @@ struct pd_sim {
                   const ClassStarts& cs, int numColors, int cap) {
     // (a part of fewer than ~100 bodies is all boundary: packed rings, 35 contacts a body)
     // Up to partRows x PT_SINGLE rows one workgroup holds a colour's rows at once and no states
-    // travel (300 spheres, 570 + 1,010 rows: 0.49 ms per substep in one workgroup, 0.66 in
-    // several); beyond, a chunk of each colour per workgroup is best (9,001 spheres at 160 / 256 /
-    // 384 / 640 rows per workgroup: 1.12 / 1.09 / 1.15 / 1.30 ms).
+    // travel (300 spheres, 577 velocity rows: 0.50 ms of velocity loops per substep in one
+    // workgroup, 0.61 in several); beyond, a chunk of each colour per workgroup is best (9,001
+    // spheres at 160 / 256 / 384 / 640 rows per workgroup: 1.12 / 1.09 / 1.15 / 1.30 ms).
     const int parts = rows <= PT_SINGLE * partRows
                           ? 1
                           : (int)std::min<long>(std::min<long>(partMax, 1 + ids / partBodies),
@@ -3291,7 +3292,8 @@ void writeLammps(const std::string& filename, int step, const double* pos, const
 // ---- autotuner (no reference counterpart) -------------------------------------------------
 // Chooses the performance knobs of a simulation by timing its own substeps: the candidate-list
 // skin (candidate_skin_permille), the largest sweep loop run inside one workgroup
-// (block_solver_rows), LDS staging of the one-workgroup velocity loop (velocity_loop_lds) and the
+// (block_solver_rows; 0 also leaves out the partition), the velocity loop over a partition of the
+// bodies (velocity_loop_lds) and the
 // register budget of the per-colour PGS sweep (vsweep_waves: 3 or 4 waves per SIMD).
 // None of them changes a result, so the trials step the simulation itself.  Coordinate descent
 // from the current setting: each knob's values are tried in turn (one untimed substep after a
