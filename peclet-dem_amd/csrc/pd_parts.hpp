@@ -197,22 +197,23 @@ __device__ __forceinline__ void partExtent(const double (&x)[3], double* lo, dou
   }
   __syncthreads();
 }
-// Clears the counters; the first workgroup lays the cells over the rows' bodies: over the
-// quantiles above and 0.15 of their distance on either side, within the broadphase grid's box.
-// Bodies outside fall into the outermost cells.  (The halvings are few and would be spent on the
-// way to one distant body: with 9,001 spheres, one of them a thousand bed widths away, the velocity
-// loops took 1.26 ms over the whole box and take 0.36 over the quantiles.)
-__global__ __launch_bounds__(TPB) void k_part_begin(PartList Q, const Grid* box, const int2* ends,
-                                                    const double4* pos, int ids, int rows, int cells,
-                                                    int levels) {
-  static_assert(TPB == 256, "16 groups of 16 samples");
+__global__ __launch_bounds__(TPB) void k_part_begin(PartList Q, int ids, int cells) {
   const int i = gtid();
   if (i < ids) Q.mask[i] = 0ull;
   if (i == 0) *Q.listCnt = 0;
   if (i < cells) Q.hist[i] = 0;
   if (i < Q.numParts) Q.partCnt[i] = 0;
   if (i < Q.numParts * Q.numColors * 2) Q.bktCnt[i] = 0;
-  if (blockIdx.x != 0) return;
+}
+// One workgroup lays the cells: over the quantiles above and 0.15 of their distance on either side,
+// within the broadphase grid's box.  Bodies outside fall into the outermost cells.  (The halvings
+// are few and would be spent on the way to one distant body: with 9,001 spheres, one of them a
+// thousand bed widths away, the velocity loops took 1.26 ms over the whole box and take 0.36 over
+// the quantiles.)
+__device__ __forceinline__ void partLayCells(const PartList& Q, const Grid* box, const int2* ends,
+                                             const double4* pos, int rows, int levels) {
+  static_assert(TPB == 256, "16 groups of 16 samples");
+  const int i = (int)threadIdx.x;
   __shared__ double lo[3], hi[3];
   const Grid b = *box;
   const double e[3] = {b.h * b.dim[0], b.h * b.dim[1], b.h * b.dim[2]};
@@ -275,9 +276,15 @@ __device__ __forceinline__ int classOf(const ClassStarts& cs, int numColors, int
   }
   return lo;
 }
+// the colours of each body's rows; the first workgroup lays the cells meanwhile
 __global__ __launch_bounds__(TPB) void k_part_colours(PartList Q, const int2* ends, ClassStarts cs,
-                                                      int rows) {
-  const int k = gtid();
+                                                      int rows, const Grid* box, const double4* pos,
+                                                      int levels) {
+  if (blockIdx.x == 0) {
+    partLayCells(Q, box, ends, pos, rows, levels);
+    return;
+  }
+  const int k = gtid() - TPB;
   if (k >= rows) return;
   const int2 ab = ends[k];
   const unsigned long long bit = 1ull << classOf(cs, Q.numColors, k);

@@ -2059,9 +2059,8 @@ struct pd_sim {
     J.sync.ensure(2 * PT_MAX_PARTS + (PT_MAX_PARTS + 1 + 3) / 4, st);
     if (parts > 1) J.lines.ensure((size_t)rows * 4 * (VEL ? 6 : 3), st);
     if (parts > 1) {  // (a loop of one workgroup builds its partition itself)
-      k_part_begin<<<nblk(std::max(std::max(ids, cells), 2 * bkts)), TPB, 0, st>>>(
-          Q, gridD.p, ends, posOf, ids, rows, cells, levels);
-      k_part_colours<<<nblk(rows), TPB, 0, st>>>(Q, ends, cs, rows);
+      k_part_begin<<<nblk(std::max(std::max(ids, cells), 2 * bkts)), TPB, 0, st>>>(Q, ids, cells);
+      k_part_colours<<<1 + nblk(rows), TPB, 0, st>>>(Q, ends, cs, rows, gridD.p, posOf, levels);
       k_part_hist<<<nblk(ids), TPB, 0, st>>>(Q, posOf, ids);
       scanQuiet(Q.hist, Q.cellStart, cells);
       k_part_assign<<<(ids + 1023) / 1024, 1024, 0, st>>>(Q, posOf, ids, cells);
