@@ -407,8 +407,10 @@ def test_candidate_list_left_out_after_failures(hip_lib, skin):
     # reuse, the substeps that go without one, and the next list
     h, _ = run_pair("bed_periodic", 300, 50, tuning={"candidate_skin_permille": skin})
     paths = h.debug_paths()
-    assert paths["list_rebuilt"] == 3 and paths["list_left_out"] >= 33
+    # (after two lists in vain 8 substeps without, then 16, 32: all 50 in vain, 2 + 2 lists)
+    assert paths["list_rebuilt"] >= 4 and paths["list_left_out"] >= 8
     assert (paths["list_reused"] > 0) == (skin == 100)
+    assert skin == 100 or paths["list_rebuilt"] == 4
 
 
 @pytest.mark.gpu
@@ -423,12 +425,12 @@ def test_candidate_list_returns_after_a_change(hip_lib, change):
     scene["vel"] = scene["vel"] + np.array([3.0, 2.0, 0.0])
     h = apply_scene(Simulation(300), scene)
     h.set_tuning("candidate_skin_permille", 1)
-    for _ in range(16):
+    for _ in range(24):  # (two lists in vain, eight substeps without, a third, sixteen without)
         h.step(scene["dt"])
-        if h.debug_paths()["list_left_out"] >= 2:
+        if h.debug_paths()["list_left_out"] >= 10:
             break
     before = h.debug_paths()
-    assert before["list_left_out"] >= 2
+    assert before["list_left_out"] >= 10
     if change == "autotune":
         cfg, ms = h.autotune(scene["dt"], substeps=2, use_cache=False)
         # every trial with a skin of its own builds one: the current, four tried, the choice
