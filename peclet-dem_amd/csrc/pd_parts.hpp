@@ -13,8 +13,8 @@
 //     workgroup sends a body's state as soon as the body's previous row is done, usually some
 //     colours before the other needs it, and there is no barrier over the grid;
 //   * two lanes evaluate a row, one for each of its bodies, exchanging what the row's impulses need
-//     of both: a colour pass of a part is a few waves' dependent FP64 arithmetic, and this halves
-//     it (560 -> 330 operations per wave);
+//     of both: a colour pass of a part is a few waves' dependent FP64 arithmetic, and this shortens
+//     it;
 //   * a workgroup's rows lie in colour order in chunks of one wave, and a wave loads its next chunk
 //     as soon as it has finished one, so that the latency passes during the colours in between (a
 //     wave with one chunk never loads it again).
@@ -38,11 +38,13 @@
 // every wait ends, since a workgroup never leaves before the loop does; the waits are bounded all
 // the same, in polls and not by a clock (a process may be suspended for any time, and its polls
 // with it), and a wait that runs out raises an error on the host.
-// Bound: a colour pass is one row's dependent arithmetic, ~430 FP64 operations at 5-8 clocks plus
-// the loads of its bodies from LDS, 1.7-2 us, and for a row between parts what the hop leaves of
-// ~1.5 us; ~200 velocity and ~110 position passes make a substep.  Substeps of resting beds, MI355X,
-// launches per colour or one workgroup (before) -> this: 4,099 spheres 2.31 -> 0.90 ms, 9,001
-// 4.03 -> 0.99 ms, 100,003 3.14 -> 2.12 ms; 60,013 raining 2.67 -> 1.41 ms.
+// Bound: below ~50k rows by a colour pass's chain, the loads of a row's bodies, its dependent FP64
+// arithmetic and for a row between parts the hop: 4,099 resting spheres 631 us for ~175 velocity
+// passes and 203 us for 108 position passes (kernel trace, 3.6 and 1.9 us each).  Above by the rows'
+// constants, gathered anew in every pass: 100,003 spheres 3.5 and 4.0 TB/s, 1M poured 5.0 and 5.2.
+// Substeps of resting beds, MI355X, launches per colour or one workgroup (before) -> this: 4,099
+// spheres 2.31 -> 0.90 ms, 9,001 4.03 -> 0.99 ms, 100,003 3.14 -> 2.12 ms; 60,013 raining 2.67 ->
+// 1.41 ms.
 #pragma once
 
 #include "pd_kernels.hpp"
