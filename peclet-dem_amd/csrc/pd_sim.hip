@@ -1977,7 +1977,7 @@ struct pd_sim {
   // bed, launches / partition: 0.45M rows 2.54 / 2.13, 0.93M 4.00 / 3.79, 1.05M 4.24 / 4.41; ms per
   // substep of 1M spheres, 1.96M rows 16.0 / 17.0).
   static constexpr long PARTS_V_ROWS = 1000000;
-  // Position rows: the two forms are within a tenth of each other from half a million rows on, up
+  // Position rows: the two forms are within an eighth of each other from half a million rows on, up
   // to this many (ms of position loops per substep, launches / partition: 0.30M rows 0.52 / 0.46,
   // 0.60M 0.69 / 0.72, 0.90M 0.90 / 0.88, 1.2M 1.04 / 1.18, 1.5M 1.35 / 1.33, 3.1M 2.71 / 2.62,
   // 4.2M 3.37 / 3.35; 6M 4.73 / 5.54, 12M 8.98 / 12.94).
