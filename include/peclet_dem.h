@@ -295,7 +295,8 @@ int pd_set_timing(pd_sim* s, int level);
  * the free device memory; 0 replays the segment for its states and each substep again right
  * before its reverse; "side_stream_min_contacts" (default 0): contact lists of at least that
  * many contacts are coloured on the simulation's second stream, beside the velocity stage,
- * shorter ones on its main stream.  Results do not depend on any of them. */
+ * shorter ones on its main stream.  Results do not depend on any of them ("partition_wait_polls"
+ * and "partition_absent" can make a step fail). */
 int pd_set_tuning(pd_sim* s, const char* name, long value);
 /* Autotuner (no reference counterpart): chooses candidate_skin_permille, block_solver_rows,
  * velocity_loop_lds and vsweep_waves for this simulation by timing its own substeps (coordinate
